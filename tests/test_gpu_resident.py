@@ -1,0 +1,202 @@
+"""The resident integrator (one kernel for many attempts) against the captured
+attempt (a graph of kernels per attempt).
+
+Both call the same element functions and sum each row in the same order, so a
+run has to give the same bits on either: state, times, step lengths, maxima,
+error ratios, rejections and observed entries.  A run that also logs an
+observation point's displacement takes the captured attempt; without it, a
+kernel of this size takes the resident one.
+
+Sizes: one element; one block and the first two-block size; blocks' shares that
+do not divide; rows that do not fit the blocks' LDS; every model, with volumes;
+the reduced forms of K; a run split into calls; an end time, a step limit and a
+run that ends in an error.
+"""
+import numpy as np
+import pytest
+
+from unicycle_amd import PREC_MIXED, PREC_SPLIT_BF16, UcyError, configs
+
+pytestmark = pytest.mark.gpu
+
+HUGE = 1.0e30
+
+
+def _segments(make, n):
+    eng = make()
+    w = np.full(n, 400.0)
+    x = np.zeros((n, 3))
+    x[:, 2] = 400.0 * np.arange(n)
+    one = np.ones(n)
+    z = (np.arange(n) + 0.5) / n
+    b = np.where((z > 0.2) & (z < 0.8), 0.014, 0.006)
+    eng.set_antiplane(30e3, x, w, np.full(n, np.pi / 2))
+    eng.set_friction(1e-9 * one, 0 * one, 0.6 * one, 100.0 * one, 0.010 * one, b, 0.01 * one,
+                     1e-6 * one, 5.0 * one)
+    return eng
+
+
+def _thrust(make, nx, nz):
+    m = configs.thrust_fault(nx=nx, nz=nz, ellipse=None)
+    eng = make()
+    eng.set_elastic(m.lambda_, m.mu)
+    eng.set_rectangles(*m.geometry())
+    eng.set_friction(*m.friction())
+    return eng
+
+
+def _volumes(make, nx, nz, v):
+    eng = _thrust(make, nx, nz)
+    g = configs.volume_grid(nx=v[0], ny=v[1], nz=v[2], top=60e3)
+    eng.set_volumes(*g.geometry())
+    eng.set_rheology(*g.rheology())
+    return eng
+
+
+def _antiplane_volumes(make, n, n2, n3):
+    m = configs.antiplane_viscous(n, n2, n3)
+    f = m.fault
+    eng = make()
+    eng.set_antiplane(f.mu, f.x, f.width, f.dip)
+    eng.set_antiplane_volumes(m.vx, m.thickness, m.vwidth, m.vdip)
+    eng.set_friction(*f.friction())
+    eng.set_rheology(*m.rheology())
+    return eng
+
+
+def _planestrain(make, n, n2=0, n3=0):
+    m = configs.planestrain_viscous(n, n2, n3) if n2 else None
+    f = m.fault if m else configs.planestrain_fault(n)
+    eng = make()
+    eng.set_planestrain(f.lambda_, f.mu, f.x, f.width, f.dip)
+    if m:
+        eng.set_planestrain_volumes(m.vx, m.thickness, m.vwidth, m.vdip)
+    eng.set_friction(*f.friction())
+    if m:
+        eng.set_rheology(*m.rheology())
+    return eng
+
+
+MODELS = {
+    "antiplane-1": lambda mk: _segments(mk, 1),
+    "antiplane-2": lambda mk: _segments(mk, 2),
+    "antiplane-64": lambda mk: _segments(mk, 64),
+    "antiplane-65": lambda mk: _segments(mk, 65),
+    "antiplane-111": lambda mk: _segments(mk, 111),
+    "antiplane-850": lambda mk: _segments(mk, 850),
+    "thrust-1": lambda mk: _thrust(mk, 1, 1),
+    "thrust-44": lambda mk: _thrust(mk, 11, 4),
+    "thrust-45": lambda mk: _thrust(mk, 9, 5),
+    "thrust-247": lambda mk: _thrust(mk, 19, 13),
+    "thrust-1081": lambda mk: _thrust(mk, 47, 23),
+    "thrust-2816": lambda mk: _thrust(mk, 64, 44),
+    "antiplane-volumes": lambda mk: _antiplane_volumes(mk, 41, 5, 7),
+    "planestrain-51": lambda mk: _planestrain(mk, 51),
+    "planestrain-volumes": lambda mk: _planestrain(mk, 24, 4, 3),
+    "volumes": lambda mk: _volumes(mk, 7, 5, (3, 3, 2)),
+    "volumes-large": lambda mk: _volumes(mk, 13, 7, (5, 5, 4)),
+}
+
+
+def _start(eng):
+    y = eng.initStateVector()
+    rng = np.random.default_rng(3)
+    if eng.antiplane:
+        y[3:4 * eng.np:4] += 0.01 * rng.standard_normal(eng.np)
+    elif eng.planestrain:
+        y[4:5 * eng.np:5] += 0.01 * rng.standard_normal(eng.np)
+    else:
+        y[6:7 * eng.np:7] += 0.01 * rng.standard_normal(eng.np)
+        y[4:7 * eng.np:7] = rng.uniform(0.1, 1.0, eng.np)
+    return y
+
+
+def _same(a, b):
+    assert (a.steps, a.attempts, a.rhs_evals) == (b.steps, b.attempts, b.rhs_evals)
+    assert a.time == b.time and a.dt_next == b.dt_next and a.vmax == b.vmax
+    for k in ("y", "t_log", "dt_log", "vmax_log", "errmax_log", "reject_log", "emax_log", "obs_y",
+              "obs_dydt"):
+        assert np.array_equal(getattr(a, k), getattr(b, k)), k
+
+
+@pytest.mark.parametrize("name", MODELS)
+def test_same_bits_as_the_captured_attempt(engine_factory, name):
+    eng = MODELS[name](engine_factory)
+    eng.buildG()
+    y = _start(eng)
+    eng.buildO(np.array([[1e3, 2e3, 0.0]]))
+    obs = [0, y.size // 2, y.size - 1]
+    kw = dict(max_steps=120, log_cap=120, history=True, observe=obs)
+    _same(eng.integrate(y, HUGE, **kw), eng.integrate(y, HUGE, displacement=True, **kw))
+    eng.close()
+
+
+@pytest.mark.parametrize("name", ["thrust-45", "thrust-247", "volumes"])
+@pytest.mark.parametrize("precision", [PREC_MIXED, PREC_SPLIT_BF16])
+def test_reduced_precision(engine_factory, name, precision):
+    eng = MODELS[name](engine_factory)
+    eng.buildG(precision)
+    y = _start(eng)
+    eng.buildO(np.array([[1e3, 2e3, 0.0]]))
+    kw = dict(max_steps=60, log_cap=60, history=True, observe=[0, 3], max_step=1e6)
+    _same(eng.integrate(y, HUGE, **kw), eng.integrate(y, HUGE, displacement=True, **kw))
+    eng.close()
+
+
+def test_largest(engine_factory):
+    """No row fits LDS beside the slip rates."""
+    eng = _thrust(engine_factory, 128, 64)
+    eng.buildG(PREC_MIXED)
+    y = _start(eng)
+    eng.buildO(np.array([[1e3, 2e3, 0.0]]))
+    kw = dict(max_steps=12, log_cap=12, history=True)
+    a, b = eng.integrate(y, HUGE, **kw), eng.integrate(y, HUGE, displacement=True, **kw)
+    assert np.array_equal(a.y, b.y) and np.array_equal(a.errmax_log, b.errmax_log)
+    eng.close()
+
+
+@pytest.mark.parametrize("n", [1, 111])
+def test_a_run_in_pieces(engine_factory, n):
+    eng = _segments(engine_factory, n)
+    eng.buildG()
+    y = _start(eng)
+    whole = eng.integrate(y, HUGE, max_steps=90, log_cap=90)
+    t, dt, times = 0.0, 1e-3, []
+    for k in (1, 2, 40, 47):
+        r = eng.integrate(y, HUGE, dt0=dt, max_steps=k, log_cap=k, t0=t)
+        y, t, dt = r.y, r.time, r.dt_next
+        times.append(r.t_log)
+    assert np.array_equal(np.concatenate(times), whole.t_log)
+    assert np.array_equal(y, whole.y)
+    eng.close()
+
+
+def test_more_attempts_than_one_launch_takes(engine_factory):
+    """A launch ends after 2000 attempts at the latest, also between the
+    rejected attempts of a step."""
+    eng = _segments(engine_factory, 1)
+    eng.set_kernel(np.array([[-7 * np.pi / 16 * 30e3 / 6e3]]))
+    y = _start(eng)
+    eng.buildO(np.array([[0.0, 1e3, 0.0]]))
+    a = eng.integrate(y, HUGE, max_steps=4500, log_cap=4500, max_step=1e7, history=True)
+    b = eng.integrate(y, HUGE, max_steps=4500, log_cap=4500, max_step=1e7, history=True,
+                      displacement=True)
+    assert a.attempts > 4000 and a.reject_log.sum() > 0
+    assert np.array_equal(a.y, b.y) and np.array_equal(a.t_log, b.t_log)
+    assert np.array_equal(a.reject_log, b.reject_log)
+    eng.close()
+
+
+def test_end_time_and_errors(engine_factory):
+    eng = _thrust(engine_factory, 9, 5)
+    eng.buildG()
+    y = _start(eng)
+    r = eng.integrate(y, 5.0e5, max_step=1e5, log_cap=100)
+    assert r.time >= 5.0e5 and r.t_log[-2] < 5.0e5
+    bad = y.copy()
+    bad[6] = np.nan
+    with pytest.raises(UcyError, match="non-finite"):
+        eng.integrate(bad, HUGE, max_steps=5)
+    again = eng.integrate(y, 5.0e5, max_step=1e5, log_cap=100)
+    assert np.array_equal(again.y, r.y)
+    eng.close()

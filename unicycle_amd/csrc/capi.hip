@@ -22,6 +22,7 @@
 #include <vector>
 #include "../../include/ucy.h"
 #include "ucy_internal.h"
+#include "resident.h"
 #include "ucy_ext.h"
 #include "ucy_ctx.h"
 
@@ -267,6 +268,7 @@ extern "C" void ucy_destroy(ucy_ctx *c)
     if (c->d_ctl) hipFree(c->d_ctl);
     if (c->h_ctl) hipHostFree(c->h_ctl);
     if (c->hook.p) hipFree(c->hook.p);
+    if (c->res.p) hipFree(c->res.p);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
 }
@@ -1649,6 +1651,91 @@ static int capture_attempt(ucy_ctx *c)
     return 0;
 }
 
+// The resident integrator's blocks, their shares and LDS (k_resident.hip), with
+// its buffers in place.  0: planned; 1: the model takes the captured attempt;
+// < 0: an error.
+//   - Share of a block: 48 KB of K, so that a stage's products (0.2 us) take
+//     less than the exchange among the blocks (1.5 us with 8, 3.8 us with 256).
+//     8 to 72 KB measure within 10 % of each other; a reduced K has fewer bytes
+//     per row and takes 16 KB (200 patches: 28 us per attempt, 35 us at 48 KB).
+//   - One block where K fits it whole, as it needs no exchange.
+//   - At most 1 GB of K in binary64 (4096 patches: 755 us per attempt, captured
+//     770 us; 8192 patches: 2985 and 2910 us, the launches no longer show) and
+//     2 GB reduced (8192 patches: 1775 and 1800 us).
+//   - Rows beyond LDS up to 64 KB per CU are left to the L2 (1600 patches 103 us,
+//     109 us if all stream; 2816 patches 368 and 353 us).
+static int plan_resident(ucy_ctx *c, const PlainDims &d, ResArgs &a, size_t &lds)
+{
+    constexpr int64_t kLds = 158 * 1024, kOneBlock = 96 * 1024, kCachedBytes = 64 * 1024;
+    const bool f64 = c->kprec == UCY_PREC_F64;
+    const int64_t m = d.m, n = d.n, entry = f64 ? 8 : 4, kShare = (f64 ? 48 : 16) * 1024;
+    const int64_t kb = m * n * entry;
+    const int ne = d.np + d.nv;
+    if (kb > (f64 ? 1ll << 30 : 2ll << 30)) return 1;
+    int64_t P = kb <= kOneBlock && ne <= 64 ? 1 : std::max<int64_t>(2, (kb + kShare - 1) / kShare);
+    P = std::max<int64_t>(P, (ne + 55) / 56);
+    P = std::min<int64_t>(P, kResMaxBlocks);
+    // element boundaries at equal numbers of rows
+    const int64_t rp = d.ps ? 2 : d.ap ? 1 : 3, rv = d.ps ? 3 : d.ap ? 2 : 6;
+    std::vector<int> bounds(P + 1);
+    int el = 0, rows = 0;
+    for (int64_t b = 0; b <= P; b++) {
+        const int64_t r = m * b / P;
+        bounds[b] = (int)(r <= rp * d.np ? (r + rp - 1) / rp
+                                         : d.np + (r - rp * d.np + rv - 1) / rv);
+        if (b == 0) continue;
+        auto row = [&](int e) { return e <= d.np ? rp * e : rp * d.np + rv * (e - d.np); };
+        el = std::max(el, bounds[b] - bounds[b - 1]);
+        rows = std::max(rows, (int)(row(bounds[b]) - row(bounds[b - 1])));
+    }
+    if (el > 64) return 1;
+    el += el & 1;
+    rows += rows & 1;
+    const int64_t other = 8 * (n + 2ll * resident_state_entries(d) * el + 2ll * rows);
+    if (other > kLds) return 1;
+    const int64_t lr = std::min<int64_t>(rows, (kLds - other) / (n * entry));
+    lds = (size_t)(other + lr * n * entry);
+    const size_t hb = 64, bb = 8 * (kResMaxBlocks / 2 + 1);
+    a.xbytes = 8 * 4 * (3 * (size_t)P + (size_t)n);
+    int rc = ensure_buf(c, c->res, hb + bb + a.xbytes);
+    if (rc) return rc;
+    char *p = (char *)c->res.p;
+    a.d = d;
+    a.K = KOperand{c->K, c->Kp, c->Krs, c->kprec};
+    a.fr = c->d_fr;
+    a.rh = c->d_rh;
+    a.b = c->rb;
+    a.ctl = c->d_ctl;
+    a.head = (ResHead *)p;
+    a.bounds = (const int *)(p + hb);
+    a.red = (unsigned long long *)(p + hb + bb);
+    a.v = a.red + 4 * 3 * P;
+    a.P = (int)P;
+    a.threads = P == 1 && m <= 8 ? 128 : kResThreads;
+    a.el_max = el;
+    a.rows_max = rows;
+    a.rows_lds = (int)lr;
+    a.rows_cached = (int)(lr + kCachedBytes / (n * entry));
+    // launches of some 30 ms: 20 us and K's reading time per attempt
+    const double us = 20.0 + (double)kb / 1.0e6;
+    a.max_attempts = (int)std::max(16.0, std::min(2000.0, 30000.0 / us));
+    HIPCHK(hipMemcpyAsync((void *)a.bounds, bounds.data(), sizeof(int) * (P + 1),
+                          hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));   // bounds is on this call's stack
+    return 0;
+}
+
+// one launch of the resident integrator, the control block read back
+static int run_resident(ucy_ctx *c, const ResArgs &a, size_t lds)
+{
+    HIPCHK(hipMemsetAsync(a.head, 0, sizeof(ResHead), c->stream));
+    HIPCHK(hipMemsetAsync(a.red, 0xff, a.xbytes, c->stream));
+    HIPCHK(launch_resident(c->stream, a, lds));
+    HIPCHK(hipMemcpyAsync(c->h_ctl, c->d_ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return 0;
+}
+
 extern "C" int ucy_integrate(ucy_ctx *c, double *y, double interval, double dt0,
                              int64_t max_steps, double epsilon, double max_step, double *t_log,
                              double *dt_log, double *vmax_log, int64_t log_cap,
@@ -1763,7 +1850,31 @@ extern "C" int ucy_integrate_ex(ucy_ctx *c, double *y, double t0, double interva
     h.log_cap = cap;
     HIPCHK(hipMemcpyAsync(c->d_ctl, &h, sizeof(Control), hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(b.y, y, sizeof(double) * d.dim, hipMemcpyHostToDevice, c->stream));
-    rc = capture_attempt(c);
+    ResArgs ra{};
+    size_t res_lds = 0;
+    rc = want_disp ? 1 : plan_resident(c, d, ra, res_lds);
+    bool resident = rc == 0;
+    if (rc > 0) rc = capture_attempt(c);
+    auto w0 = std::chrono::steady_clock::now();
+    int batch = 16;
+    while (rc == 0) {
+        if (resident) {
+            const long long before = h.attempts;
+            rc = run_resident(c, ra, res_lds);
+            if (rc || h.done) break;
+            // the blocks found no room together: the captured attempt goes on
+            if (h.attempts == before) {
+                resident = false;
+                rc = capture_attempt(c);
+            }
+            continue;
+        }
+        for (int i = 0; i < batch; i++) HIPCHK(hipGraphLaunch(c->graph, c->stream));
+        HIPCHK(hipMemcpyAsync(c->h_ctl, c->d_ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        if (h.done) break;
+        if (batch < 256) batch *= 2;
+    }
     if (rc) {
         if (d_log) hipFree(d_log);
         if (d_oidx) {
@@ -1778,15 +1889,6 @@ extern "C" int ucy_integrate_ex(ucy_ctx *c, double *y, double t0, double interva
         b.O = nullptr;
         b.disp = b.disp_f = b.disp_l = nullptr;
         return rc;
-    }
-    auto w0 = std::chrono::steady_clock::now();
-    int batch = 16;
-    for (;;) {
-        for (int i = 0; i < batch; i++) HIPCHK(hipGraphLaunch(c->graph, c->stream));
-        HIPCHK(hipMemcpyAsync(c->h_ctl, c->d_ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        if (h.done) break;
-        if (batch < 256) batch *= 2;
     }
     // the last accepted step (later attempts commit at their start)
     launch_commit(c->stream, d.dim, b, c->d_ctl);
@@ -1826,8 +1928,8 @@ extern "C" int ucy_integrate_ex(ucy_ctx *c, double *y, double t0, double interva
     }
     HIPCHK(hipStreamSynchronize(c->stream));
     if (d_log) {
-        // the graph refers to the log buffers; drop it with them
-        hipGraphExecDestroy(c->graph);
+        // a captured attempt refers to the log buffers; drop it with them
+        if (c->graph) hipGraphExecDestroy(c->graph);
         c->graph = nullptr;
         HIPCHK(hipFree(d_log));
         b.tlog = b.dtlog = b.vlog = b.elog = b.rlog = b.emlog = nullptr;
@@ -1855,6 +1957,7 @@ extern "C" int ucy_integrate_ex(ucy_ctx *c, double *y, double t0, double interva
     }
     if (h.error == 1) return fail(c, UCY_ERR_UNDERFLOW, "stepsize underflow in RKQS");
     if (h.error == 2) return fail(c, UCY_ERR_NONFINITE, "non-finite error norm");
+    if (h.error == 3) return fail(c, UCY_ERR_HIP, "resident integrator: a block did not answer");
     return UCY_OK;
 }
 

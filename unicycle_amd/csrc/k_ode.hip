@@ -11,327 +11,9 @@
 // the run is done, so a captured attempt can be replayed any number of times.
 #include <hip/hip_runtime.h>
 #include "../../include/ucy.h"
-#include "ucy_internal.h"
+#include "ode_dev.h"
 
 namespace ucy {
-
-// ratestate.f90:130 lg10=LOG(1.d1)
-__constant__ const double kLg10 = 2.302585092994045684;
-
-// Cash-Karp tableau (ode45.f90:126-134)
-#define B21 0.2
-#define B31 (3.0 / 40.0)
-#define B32 (9.0 / 40.0)
-#define B41 0.3
-#define B42 (-0.9)
-#define B43 1.2
-#define B51 (-11.0 / 54.0)
-#define B52 2.5
-#define B53 (-70.0 / 27.0)
-#define B54 (35.0 / 27.0)
-#define B61 (1631.0 / 55296.0)
-#define B62 (175.0 / 512.0)
-#define B63 (575.0 / 13824.0)
-#define B64 (44275.0 / 110592.0)
-#define B65 (253.0 / 4096.0)
-#define C1 (37.0 / 378.0)
-#define C3 (250.0 / 621.0)
-#define C4 (125.0 / 594.0)
-#define C6 (512.0 / 1771.0)
-#define DC1 (C1 - 2825.0 / 27648.0)
-#define DC3 (C3 - 18575.0 / 48384.0)
-#define DC4 (C4 - 13525.0 / 55296.0)
-#define DC5 (-277.0 / 14336.0)
-#define DC6 (C6 - 0.25)
-
-__device__ __forceinline__ unsigned long long dbits(double x)
-{
-    return (unsigned long long)__double_as_longlong(x);
-}
-
-// ---------------------------------------------------------------------------
-// pre-pass for one patch (ratestate.f90:683-702) and one volume
-// (viscouscycles.f90:940-995)
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ double patch_prepass(const double *p, const Friction &f, double *dp,
-                                                double *vp)
-{
-    const double rake = atan2(p[3], p[2]);
-    const double velocity = exp(p[6] * kLg10);
-    const double vs = velocity * cos(rake), vd = velocity * sin(rake);
-    dp[0] = vs;
-    dp[1] = vd;
-    vp[0] = vs - f.vplc;
-    vp[1] = vd - f.vpls;
-    return velocity;
-}
-
-// 2-D antiplane patch (fortran/2d/antiplane/src/ratestate.f90:660-677): slip
-// rate V, v = V - Vpl (vplc holds Vpl)
-__device__ __forceinline__ double ap_prepass(const double *p, const Friction &f, double *dp,
-                                             double *vp)
-{
-    const double velocity = exp(p[3] * kLg10);
-    dp[0] = velocity;
-    vp[0] = velocity - f.vplc;
-    return velocity;
-}
-
-// ratestate.f90 (2-D antiplane):698-722
-__device__ __forceinline__ void ap_postpass(const double *p, const Friction &f, double t,
-                                            double *dp)
-{
-    const double velocity = exp(p[3] * kLg10);
-    dp[2] = (exp(-p[2] * kLg10) - velocity / f.L) / kLg10;
-    const double dtau = t;
-    dp[3] = (dtau - f.b * f.sig * dp[2] * kLg10) / (f.a * f.sig + f.damping * velocity) / kLg10;
-    dp[1] = dtau - f.damping * velocity * dp[3] * kLg10;
-}
-
-// 2-D plane-strain patch (fortran/2d/planestrain/src/ratestate.f90:692-712):
-// dip-slip rate V, v = V - Vpl (vplc holds Vpl)
-__device__ __forceinline__ double ps_prepass(const double *p, const Friction &f, double *dp,
-                                             double *vp)
-{
-    const double velocity = exp(p[4] * kLg10);
-    dp[0] = velocity;
-    vp[0] = velocity - f.vplc;
-    return velocity;
-}
-
-// ratestate.f90 (2-D plane strain):723-750: the dip traction drives the
-// friction law at the constant normal stress sig; the normal traction rate is
-// integrated as is
-__device__ __forceinline__ void ps_postpass(const double *p, const Friction &f, const double *t,
-                                            double *dp)
-{
-    const double velocity = exp(p[4] * kLg10);
-    dp[3] = (exp(-p[3] * kLg10) - velocity / f.L) / kLg10;
-    const double dtau = t[0];
-    const double sigma = f.sig;
-    dp[4] = (dtau - f.b * sigma * dp[3] * kLg10) / (f.a * sigma + f.damping * velocity) / kLg10;
-    dp[1] = dtau - f.damping * velocity * dp[4] * kLg10;
-    dp[2] = t[1];
-}
-
-// 2-D antiplane volume (fortran/2d/antiplane/src/viscouscycles.f90:846-877):
-// state [e12, e13, s12, s13]; strain rate eII s with
-// eII = gammadot0 (sII/Gm)^(n-1) / Gm exp(-Q/(R To)), v = that less the
-// background rate; returns the strain-rate norm (eMax of :869)
-__device__ __forceinline__ double ap_volume_prepass(const double *q, const Rheology &r, double *dq,
-                                                    double *vq)
-{
-    const double s12 = q[2], s13 = q[3];
-    const double sII = sqrt(s12 * s12 + s13 * s13);
-    const double eII = r.gammadot0 * pow(sII / r.Gm, r.npower - 1.0) / r.Gm * r.arr;
-    const double e12 = eII * s12, e13 = eII * s13;
-    dq[0] = e12;
-    dq[1] = e13;
-    vq[0] = e12 - r.ebg[1];
-    vq[1] = e13 - r.ebg[2];
-    return sqrt(e12 * e12 + e13 * e13);
-}
-
-// 2-D plane-strain volume (fortran/2d/planestrain/src/viscouscycles.f90:
-// 929-967): state [e22, e23, e33, s22, s23, s33]; with the 2-D deviatoric
-// stress s' (p = (s22 + s33) / 2), strain rate eII s' with
-// eII = gammadot0 sII^(n-1) exp(-Q/(R To)); v = (that - the background
-// rate) 1e3, as K's volume columns are strains of 1e-3; returns the
-// strain-rate norm (eMax of :962)
-__device__ __forceinline__ double ps_volume_prepass(const double *q, const Rheology &r, double *dq,
-                                                    double *vq)
-{
-    const double s22 = q[3], s23 = q[4], s33 = q[5];
-    const double p = (s22 + s33) / 2.0;
-    const double s22p = s22 - p, s33p = s33 - p;
-    const double sII = sqrt((s22p * s22p + 2.0 * (s23 * s23) + s33p * s33p) / 2.0);
-    const double eII = r.gammadot0 * pow(sII, r.npower - 1.0) * r.arr;
-    const double e22 = eII * s22p, e23 = eII * s23, e33 = eII * s33p;
-    dq[0] = e22;
-    dq[1] = e23;
-    dq[2] = e33;
-    vq[0] = (e22 - r.ebg[3]) * 1e3;
-    vq[1] = (e23 - r.ebg[4]) * 1e3;
-    vq[2] = (e33 - r.ebg[5]) * 1e3;
-    return sqrt((e22 * e22 + 2.0 * (e23 * e23) + e33 * e33) / 2.0);
-}
-
-__device__ __forceinline__ void volume_prepass(const double *q, const Rheology &r, double *dq,
-                                               double *vq)
-{
-    double s11 = q[6], s12 = q[7], s13 = q[8], s22 = q[9], s23 = q[10], s33 = q[11];
-    const double p = (s11 + s22 + s33) / 3.0;
-    s11 = s11 - p;
-    s22 = s22 - p;
-    s33 = s33 - p;
-    const double sII = sqrt((s11 * s11 + 2.0 * (s12 * s12) + 2.0 * (s13 * s13) + s22 * s22
-                             + 2.0 * (s23 * s23) + s33 * s33) / 2.0);
-    const double eII = r.gammadot0 * pow(sII, r.npower - 1.0);
-    const double e[6] = {0.0 + eII * s11, 0.0 + eII * s12, 0.0 + eII * s13,
-                         0.0 + eII * s22, 0.0 + eII * s23, 0.0 + eII * s33};
-#pragma unroll
-    for (int k = 0; k < 6; k++) {
-        dq[k] = e[k];
-        vq[k] = e[k] - r.ebg[k];
-    }
-}
-
-// post-pass for one patch (ratestate.f90:747-771)
-__device__ __forceinline__ void patch_postpass(const double *p, const Friction &f, const double *t,
-                                               double *dp)
-{
-    const double rake = atan2(p[3], p[2]);
-    const double velocity = exp(p[6] * kLg10);
-    const double cr = cos(rake), sr = sin(rake);
-    dp[5] = (exp(-p[5] * kLg10) - velocity / f.L) / kLg10;
-    const double dtau = t[0] * cr + t[1] * sr;
-    dp[6] = (dtau - f.b * f.sig * dp[5] * kLg10) / (f.a * f.sig + f.damping * velocity) / kLg10;
-    const double correction = f.damping * velocity * dp[6] * kLg10;
-    dp[2] = t[0] - correction * cr;
-    dp[3] = t[1] - correction * sr;
-    dp[4] = t[2];
-}
-
-__device__ __forceinline__ int elem_state_off(const PlainDims &d, int e)
-{
-    if (d.ps) return e < d.np ? 5 * e : 5 * d.np + 6 * (e - d.np);
-    if (d.ap) return 4 * e;
-    return e < d.np ? 7 * e : 7 * d.np + 12 * (e - d.np);
-}
-__device__ __forceinline__ int elem_v_off(const PlainDims &d, int e)
-{
-    if (d.ps) return e < d.np ? e : d.np + 3 * (e - d.np);
-    if (d.ap) return e < d.np ? e : d.np + 2 * (e - d.np);
-    return e < d.np ? 2 * e : 2 * d.np + 6 * (e - d.np);
-}
-__device__ __forceinline__ int elem_row_off(const PlainDims &d, int e)
-{
-    if (d.ps) return e < d.np ? 2 * e : 2 * d.np + 3 * (e - d.np);
-    if (d.ap) return e < d.np ? e : d.np + 2 * (e - d.np);
-    return e < d.np ? 3 * e : 3 * d.np + 6 * (e - d.np);
-}
-// state entries and slip-rate entries of element e
-__device__ __forceinline__ int elem_nstate(const PlainDims &d, int e)
-{
-    return d.ps ? (e < d.np ? 5 : 6) : d.ap ? 4 : (e < d.np ? 7 : 12);
-}
-__device__ __forceinline__ int elem_nv(const PlainDims &d, int e)
-{
-    return d.ps ? (e < d.np ? 1 : 3) : d.ap ? (e < d.np ? 1 : 2) : (e < d.np ? 2 : 6);
-}
-
-// ---------------------------------------------------------------------------
-// wave-level dot products of NR rows of K with v; one wavefront per element
-// ---------------------------------------------------------------------------
-// K is streamed once per RHS: non-temporal loads keep it from evicting v and
-// the state from the caches
-typedef double f64x2 __attribute__((ext_vector_type(2)));
-
-template <int NR>
-__device__ __forceinline__ void wave_rows_dot(const double *__restrict__ K, int64_t row0, int n,
-                                              const double *__restrict__ v, int lane, double acc[NR])
-{
-#pragma unroll
-    for (int r = 0; r < NR; r++) acc[r] = 0.0;
-    const int n2 = n >> 1;
-    const double2 *v2 = reinterpret_cast<const double2 *>(v);
-    const f64x2 *kr[NR];
-#pragma unroll
-    for (int r = 0; r < NR; r++) kr[r] = reinterpret_cast<const f64x2 *>(K + (row0 + r) * (int64_t)n);
-    int j = lane;
-    for (; j + 192 < n2; j += 256) {
-        double2 vv[4];
-        f64x2 kk[NR][4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) vv[u] = v2[j + 64 * u];
-#pragma unroll
-        for (int r = 0; r < NR; r++)
-#pragma unroll
-            for (int u = 0; u < 4; u++) kk[r][u] = __builtin_nontemporal_load(kr[r] + j + 64 * u);
-#pragma unroll
-        for (int r = 0; r < NR; r++)
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                acc[r] = fma(kk[r][u].x, vv[u].x, acc[r]);
-                acc[r] = fma(kk[r][u].y, vv[u].y, acc[r]);
-            }
-    }
-    for (; j < n2; j += 64) {
-        const double2 vv = v2[j];
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            const f64x2 kk = kr[r][j];
-            acc[r] = fma(kk.x, vv.x, acc[r]);
-            acc[r] = fma(kk.y, vv.y, acc[r]);
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < NR; r++) {
-        double a = acc[r];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
-        acc[r] = a;
-    }
-}
-
-// the same with the packed split-bf16 K: entry = (hi + lo) * rs[row], each
-// pair decoded exactly to binary64 and accumulated in binary64 (the GEMV is
-// bound by HBM at 4 bytes per entry, so the wider arithmetic is free)
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ double split_entry(uint32_t w)
-{
-    return (double)__uint_as_float(w & 0xFFFF0000u) + (double)__uint_as_float(w << 16);
-}
-
-template <int NR>
-__device__ __forceinline__ void wave_rows_dot_split(const uint32_t *__restrict__ Kp,
-                                                    const double *__restrict__ rs, int64_t row0,
-                                                    int n, const double *__restrict__ v, int lane,
-                                                    double acc[NR])
-{
-#pragma unroll
-    for (int r = 0; r < NR; r++) acc[r] = 0.0;
-    const int n2 = n >> 1;
-    const double2 *v2 = reinterpret_cast<const double2 *>(v);
-    const u32x2 *kr[NR];
-#pragma unroll
-    for (int r = 0; r < NR; r++) kr[r] = reinterpret_cast<const u32x2 *>(Kp + (row0 + r) * (int64_t)n);
-    int j = lane;
-    for (; j + 192 < n2; j += 256) {
-        double2 vv[4];
-        u32x2 kk[NR][4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) vv[u] = v2[j + 64 * u];
-#pragma unroll
-        for (int r = 0; r < NR; r++)
-#pragma unroll
-            for (int u = 0; u < 4; u++) kk[r][u] = __builtin_nontemporal_load(kr[r] + j + 64 * u);
-#pragma unroll
-        for (int r = 0; r < NR; r++)
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                acc[r] = fma(split_entry(kk[r][u].x), vv[u].x, acc[r]);
-                acc[r] = fma(split_entry(kk[r][u].y), vv[u].y, acc[r]);
-            }
-    }
-    for (; j < n2; j += 64) {
-        const double2 vv = v2[j];
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            const u32x2 kk = kr[r][j];
-            acc[r] = fma(split_entry(kk.x), vv.x, acc[r]);
-            acc[r] = fma(split_entry(kk.y), vv.y, acc[r]);
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < NR; r++) {
-        double a = acc[r];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
-        acc[r] = a * rs[row0 + r];
-    }
-}
 
 __global__ void __launch_bounds__(256) matvec_split_kernel(const uint32_t *__restrict__ Kp,
                                                            const double *__restrict__ rs, int m,
@@ -582,18 +264,6 @@ void launch_gemv_post(hipStream_t st, const PlainDims &d, const double *K, const
 // v2) because a wave writes the next stage's entries of its element while
 // other waves still read the current ones.  A run ends with one commit.
 // ---------------------------------------------------------------------------
-// max of the bit patterns of a wavefront's non-negative values (NaN bits
-// order above +inf), every lane active
-__device__ __forceinline__ unsigned long long wave_max_bits(unsigned long long b)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const unsigned long long c = (unsigned long long)__shfl_xor((long long)b, o, 64);
-        b = c > b ? c : b;
-    }
-    return b;
-}
-
 __global__ void start_kernel(PlainDims d, const Friction *__restrict__ fr,
                              const Rheology *__restrict__ rh, RkBuffers b, Control *ctl)
 {
@@ -650,40 +320,6 @@ void launch_start(hipStream_t st, const PlainDims &d, const Friction *fr, const 
 {
     const int ne = d.np + d.nv;
     hipLaunchKernelGGL(start_kernel, dim3((ne + 255) / 256), dim3(256), 0, st, d, fr, rh, b, ctl);
-}
-
-// intermediate state of stage s (ode45.f90:137-180), BLAS-1 order kept:
-// yrkck = B_s1*dydt; yrkck += B_sj*AKj; ytmp = yin + h*yrkck
-__device__ __forceinline__ double stage_value(int stage, double h, double y0, double k1, double k2,
-                                              double k3, double k4, double k5)
-{
-    double yr;
-    switch (stage) {
-    case 2:
-        return y0 + (h * B21) * k1;
-    case 3:
-        yr = B31 * k1;
-        yr = yr + B32 * k2;
-        return y0 + h * yr;
-    case 4:
-        yr = B41 * k1;
-        yr = yr + B42 * k2;
-        yr = yr + B43 * k3;
-        return y0 + h * yr;
-    case 5:
-        yr = B51 * k1;
-        yr = yr + B52 * k2;
-        yr = yr + B53 * k3;
-        yr = yr + B54 * k4;
-        return y0 + h * yr;
-    default:
-        yr = B61 * k1;
-        yr = yr + B62 * k2;
-        yr = yr + B63 * k3;
-        yr = yr + B64 * k4;
-        yr = yr + B65 * k5;
-        return y0 + h * yr;
-    }
 }
 
 // the input of stage `stage` (2..6) for element e and its pre-pass; the
@@ -808,62 +444,9 @@ void launch_rhs_finish(hipStream_t st, const PlainDims &d, const KOperand &K, co
         hipLaunchKernelGGL(rhs_finish_kernel<DOT_SPLIT_INC>, g, t, 0, st, d, K, fr, b, ctl);
 }
 
-// step control of RKQSm (ode45.f90:70-105) and the time update / exit test of
-// the main loop (ratestate.f90:317-326).  RKQSm is called with t0 = 0
-// (ratestate.f90:317), so its underflow test is h == 0.
 __global__ void controller_kernel(RkBuffers b, Control *ctl)
 {
-    if (ctl->done) return;
-    const double SAFETY = 0.7, PGROW = -0.2, PSHRNK = -0.15, ERRCON = 1.89e-4;
-    ctl->attempts += 1;
-    ctl->rhs_evals += ctl->need_rhs ? 6 : 5;
-    const double raw = __longlong_as_double((long long)ctl->errmax_bits);
-    if (!(raw == raw) || raw > 1.7976931348623157e308) {
-        ctl->error = 2;
-        ctl->done = 1;
-        ctl->accepted = 0;
-        return;
-    }
-    const double errmax = raw / ctl->epsilon;
-    double h = ctl->h;
-    if (errmax > 1.0) {
-        h = h * SAFETY * pow(errmax, PSHRNK);
-        ctl->h = h;
-        ctl->need_rhs = 0;
-        ctl->accepted = 0;
-        ctl->step_rejects += 1;
-        if (0.0 + h == 0.0) {
-            ctl->error = 1;
-            ctl->done = 1;
-        }
-        return;
-    }
-    double hnext = errmax > ERRCON ? SAFETY * h * pow(errmax, PGROW) : 10.0 * h;
-    if (hnext > ctl->max_step) hnext = ctl->max_step;
-    ctl->hdid = h;
-    ctl->hnext = hnext;
-    ctl->time = ctl->time + h;
-    ctl->steps += 1;
-    if (ctl->log_count < ctl->log_cap) {
-        b.tlog[ctl->log_count] = ctl->time;
-        b.dtlog[ctl->log_count] = h;
-        b.vlog[ctl->log_count] = ctl->vmax;
-        if (b.elog) {
-            b.elog[ctl->log_count] = errmax;
-            b.rlog[ctl->log_count] = (double)ctl->step_rejects;
-        }
-        if (b.emlog) b.emlog[ctl->log_count] = ctl->emax;
-        ctl->log_count += 1;
-    }
-    ctl->step_rejects = 0;
-    ctl->last_vmax = ctl->vmax;
-    ctl->vmax = 0.0;
-    ctl->emax = 0.0;
-    ctl->accepted = 1;
-    ctl->obs_pending = 1;
-    ctl->need_rhs = 1;
-    ctl->h = hnext;
-    if (ctl->interval <= ctl->time || ctl->steps >= ctl->max_steps) ctl->done = 1;
+    controller_step(b, ctl, true);
 }
 
 // the step-start state and derivative of the observed entries after an

@@ -80,6 +80,8 @@ struct ucy_ctx {
     hipGraphExec_t graph = nullptr;
     // scratch for the per-kernel hooks
     DevBuf hook;
+    // the resident integrator's exchange buffers
+    DevBuf res;
     // ensembles created on this context (destroyed with it)
     std::vector<struct ucy_ensemble *> ensembles;
 };
