@@ -4,8 +4,8 @@
 //
 // Host: per-source geometry (TD frames, vertex angles, side transforms) with
 // the C library, as DispInHalfSpace.c / StrainInHalfSpace.c form it.
-// Device: one (receiver, source) pair per lane, both unit slips per lane,
-// each receiver row written as a contiguous run of 2 doubles per lane.
+// Device: one (receiver, source) pair per lane, both unit slips per lane; 64
+// receivers of one source per wave, the rows written from LDS tiles.
 #include <hip/hip_runtime.h>
 #include <cmath>
 #include <string>
@@ -137,6 +137,7 @@ static TdSide host_side(const double PA[3], const double PB[3])
         T.trig[c][1] = co;
         T.trig[c][2] = co / s;
         T.trig[c][3] = cos(angs[c] / 2.0) / sin(angs[c] / 2.0);
+        T.trig[c][4] = 1.0 / co;
     }
     return T;
 }
@@ -203,63 +204,96 @@ __device__ __forceinline__ void tri_proj_volume(const Receiver &R, const double 
     o[5] = -c1 * dv[0] - c2 * dv[1] - c3 * dv[2];
 }
 
-template <int KIND, bool GEN>
-__global__ void __launch_bounds__(128)
-tri_rows_kernel(TriMedium M, const TriSource *__restrict__ src, int ns,
-                const Receiver *__restrict__ rcv, double *__restrict__ K, int64_t ldk,
-                int64_t row0, int64_t col0, double *s_out, double *d_out, int out_stride)
+// the per-pair hooks: one receiver, general slip vectors, one source per lane
+template <int KIND>
+__global__ void __launch_bounds__(64)
+tri_hook_kernel(TriMedium M, const TriSource *__restrict__ src, int ns,
+                const Receiver *__restrict__ rcv, double *__restrict__ out)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    const int r = blockIdx.y;
     if (s >= ns) return;
-    const Receiver R = rcv[r];
+    const Receiver R = rcv[0];
     double Ss[6], Sd[6];
-    tri_stress2<GEN>(M, src[s], R.xc[0], R.xc[1], R.xc[2], Ss, Sd);
+    tri_stress2<true>(M, src[s], R.xc[0], R.xc[1], R.xc[2], Ss, Sd);
     constexpr int NC = KIND == 0 ? 3 : 6;
-    double os[NC], od[NC];
-    if constexpr (KIND == 0) {
-        tri_proj_traction(R, Ss, os);
-        tri_proj_traction(R, Sd, od);
-    } else {
-        tri_proj_volume(R, Ss, os);
-        tri_proj_volume(R, Sd, od);
-    }
-    if (K) {
-        const int64_t base = (row0 + (int64_t)NC * r) * ldk + col0 + 2 * (int64_t)s;
+    double os[NC];
+    if constexpr (KIND == 0) tri_proj_traction(R, Ss, os);
+    else tri_proj_volume(R, Ss, os);
 #pragma unroll
-        for (int c = 0; c < NC; c++)
-            *reinterpret_cast<double2 *>(K + base + c * ldk) = make_double2(os[c], od[c]);
-    }
-    if (s_out) {
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            s_out[(int64_t)c * out_stride + s] = os[c];
-            d_out[(int64_t)c * out_stride + s] = od[c];
+    for (int c = 0; c < NC; c++) out[(int64_t)c * ns + s] = os[c];
+}
+
+// Rows of K (kind 0: 3 traction rows per receiver, kind 1: 6 volume-frame stress
+// rows) of 64 receivers against 4 * spw sources, both unit slips.
+//
+// Bound by the vector unit: 10,500 instructions per pair, 8,700 of them FP64,
+// issued in 78 % of the cycles; no memory traffic to speak of.  A wave takes one
+// source at a time for 64 receivers, so the source's 170 doubles come through
+// the scalar unit and leave the vector registers to the derivatives (368, one
+// wave per SIMD).  2952 triangles: 5.1 ms; with a source per lane 6.3 ms; with
+// full gradients in the source's frame, 512 registers and 1.2 KB of spills per
+// lane 15.5 ms.  Forming the harmonic terms once per column fits two waves per
+// SIMD with 57 registers spilled and takes 5.9 ms.  The block's tile goes
+// through LDS, so that a row is written in runs of 64 spw bytes.
+template <int KIND>
+__global__ void __launch_bounds__(256)
+tri_tile_kernel(TriMedium M, const TriSource *__restrict__ src, int ns, int spw,
+                const Receiver *__restrict__ rcv, int nr, double *__restrict__ K, int64_t ldk,
+                int64_t row0, int64_t col0)
+{
+    constexpr int NC = KIND == 0 ? 3 : 6;
+    extern __shared__ double2 tile[];   // [64 * NC][4 spw + 1]: padded against bank conflicts
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = blockIdx.y * 64, s0 = blockIdx.x * 4 * spw, pitch = 4 * spw + 1;
+    const int r = min(r0 + lane, nr - 1);
+    for (int k = 0; k < spw; k++) {
+        const int sl = w * spw + k, s = s0 + sl;
+        if (s >= ns) break;
+        double Ss[6], Sd[6], os[NC], od[NC];
+        tri_stress2<false>(M, src[s], rcv[r].xc[0], rcv[r].xc[1], rcv[r].xc[2], Ss, Sd);
+        const Receiver R = rcv[r];
+        if constexpr (KIND == 0) {
+            tri_proj_traction(R, Ss, os);
+            tri_proj_traction(R, Sd, od);
+        } else {
+            tri_proj_volume(R, Ss, os);
+            tri_proj_volume(R, Sd, od);
         }
+#pragma unroll
+        for (int c = 0; c < NC; c++) tile[(lane * NC + c) * pitch + sl] = make_double2(os[c], od[c]);
+    }
+    __syncthreads();
+    const int cols = min(4 * spw, ns - s0), rows = min(64, nr - r0) * NC;
+    for (int i = threadIdx.x; i < rows * 4 * spw; i += 256) {
+        const int row = i / (4 * spw), col = i - row * 4 * spw;
+        if (col < cols)
+            *reinterpret_cast<double2 *>(K + (row0 + (int64_t)NC * r0 + row) * ldk + col0 +
+                                         2 * (int64_t)(s0 + col)) = tile[row * pitch + col];
     }
 }
 
-// kind 0 traction rows, 1 volume-frame stress rows; gen: general slip
-// vectors (per-pair hooks) instead of unit strike / dip
-static void launch_tri_rows(hipStream_t st, const TriMedium &M, const TriSource *src, int ns,
+// kind 0 traction rows, 1 volume-frame stress rows.  A block takes 16 sources
+// (rows in runs of 256 bytes) where that leaves a block per CU and more, 4 for
+// small meshes, whose time is one pair's chain.
+static void launch_tri_tile(hipStream_t st, const TriMedium &M, const TriSource *src, int ns,
                             const Receiver *rcv, int nr, int kind, double *K, int64_t ldk,
-                            int64_t row0, int64_t col0, double *s_out, double *d_out, int stride,
-                            bool gen = false)
+                            int64_t row0, int64_t col0)
 {
     if (ns <= 0 || nr <= 0) return;
-    dim3 grid((ns + 127) / 128, nr);
-    if (kind == 0 && !gen)
-        hipLaunchKernelGGL((tri_rows_kernel<0, false>), grid, dim3(128), 0, st, M, src, ns, rcv, K,
-                           ldk, row0, col0, s_out, d_out, stride);
-    else if (kind == 0)
-        hipLaunchKernelGGL((tri_rows_kernel<0, true>), grid, dim3(128), 0, st, M, src, ns, rcv, K,
-                           ldk, row0, col0, s_out, d_out, stride);
-    else if (!gen)
-        hipLaunchKernelGGL((tri_rows_kernel<1, false>), grid, dim3(128), 0, st, M, src, ns, rcv, K,
-                           ldk, row0, col0, s_out, d_out, stride);
-    else
-        hipLaunchKernelGGL((tri_rows_kernel<1, true>), grid, dim3(128), 0, st, M, src, ns, rcv, K,
-                           ldk, row0, col0, s_out, d_out, stride);
+    const int rt = (nr + 63) / 64;
+    const int spw = (int64_t)rt * ((ns + 15) / 16) >= 512 ? 4 : 1;
+    const dim3 grid((ns + 4 * spw - 1) / (4 * spw), rt);
+    const size_t lds = sizeof(double2) * 64 * (kind == 0 ? 3 : 6) * (4 * spw + 1);
+    if (kind == 0) {
+        hipLaunchKernelGGL((tri_tile_kernel<0>), grid, dim3(256), lds, st, M, src, ns, spw, rcv, nr,
+                           K, ldk, row0, col0);
+    } else {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(tri_tile_kernel<1>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipLaunchKernelGGL((tri_tile_kernel<1>), grid, dim3(256), lds, st, M, src, ns, spw, rcv, nr,
+                           K, ldk, row0, col0);
+    }
 }
 
 static TriMedium tri_medium(double G, double lambda)
@@ -288,12 +322,9 @@ int ext_build_triangle_columns(hipStream_t st, double G, double lambda, int ntri
     }
     e = hipMemcpyAsync(dS, S.data(), sizeof(TriSource) * ntri, hipMemcpyHostToDevice, st);
     const TriMedium M = tri_medium(G, lambda);
-    for (int r0 = 0; r0 < np && e == hipSuccess; r0 += 65535)
-        launch_tri_rows(st, M, dS, ntri, d_R + r0, std::min(65535, np - r0), 0, K, ldk,
-                        3 * (int64_t)r0, col0, nullptr, nullptr, 0);
-    for (int r0 = 0; r0 < nvol && e == hipSuccess; r0 += 65535)
-        launch_tri_rows(st, M, dS, ntri, d_R + np + r0, std::min(65535, nvol - r0), 1, K, ldk,
-                        3 * (int64_t)np + 6 * (int64_t)r0, col0, nullptr, nullptr, 0);
+    if (e == hipSuccess) launch_tri_tile(st, M, dS, ntri, d_R, np, 0, K, ldk, 0, col0);
+    if (e == hipSuccess)
+        launch_tri_tile(st, M, dS, ntri, d_R + np, nvol, 1, K, ldk, 3 * (int64_t)np, col0);
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     (void)hipFree(dS);
@@ -366,27 +397,15 @@ __global__ void __launch_bounds__(128) strain_pairs_kernel(TriMedium M, const Tr
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const TriSource &T = S[i];
-    const G3 Xg = gmk(X[i], 1, 0, 0), Yg = gmk(Y[i], 0, 1, 0), Zg = gmk(Z[i], 0, 0, 1);
-    G3 us[3], ud[3];
-    double e[3][6], sg[3][6];
-    td_full2(T.full[0], Xg, Yg, Zg, M.nu, T.btd[0], T.btd[1], us, ud);   // main
-    sym_strain(us, e[0]);
-    hooke6(e[0], M.mu, M.lambda, sg[0]);
-    td_full2(T.full[1], Xg, Yg, Zg, M.nu, T.btd[0], T.btd[1], us, ud);   // image
-    sym_strain(us, e[1]);
-    hooke6(e[1], M.mu, M.lambda, sg[1]);
-    if (T.surface) {
-        e[1][4] = -e[1][4];
-        e[1][5] = -e[1][5];
-        sg[1][4] = -sg[1][4];
-        sg[1][5] = -sg[1][5];
-    }
-    td_fsc2(T, Xg, Yg, Zg, M.nu, us, ud);                                 // harmonic
-    sym_strain(us, e[2]);
-    hooke6(e[2], M.mu, M.lambda, sg[2]);
+    const double P[3] = {X[i], Y[i], Z[i]};
+    double e[2][2][6], s[6], im[6];
+    tri_strain2<true>(M, T, P, e);
+    hooke6(e[0][0], M.mu, M.lambda, s);
+    hooke6(e[1][0], M.mu, M.lambda, im);
     for (int k = 0; k < 6; k++) {
-        stress[6 * (size_t)i + k] = sg[0][k] + sg[1][k] + sg[2][k];
-        strain[6 * (size_t)i + k] = e[0][k] + e[1][k] + e[2][k];
+        const bool flip = T.surface && k >= 4;
+        stress[6 * (size_t)i + k] = s[k] + (flip ? -im[k] : im[k]);
+        strain[6 * (size_t)i + k] = e[0][0][k] + (flip ? -e[1][0][k] : e[1][0][k]);
     }
 }
 
@@ -473,13 +492,18 @@ static int tri_hook(ucy_ctx *c, int kind, const double x[3], const double sv[3],
     double *dout = nullptr;
     hipError_t e = hipMalloc((void **)&dS, sizeof(TriSource) * ns);
     if (e == hipSuccess) e = hipMalloc((void **)&dR, sizeof(Receiver));
-    if (e == hipSuccess) e = hipMalloc((void **)&dout, sizeof(double) * 2 * NC * (size_t)ns);
+    if (e == hipSuccess) e = hipMalloc((void **)&dout, sizeof(double) * NC * (size_t)ns);
     if (e == hipSuccess) e = hipMemcpyAsync(dS, S.data(), sizeof(TriSource) * ns, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(dR, &R, sizeof(Receiver), hipMemcpyHostToDevice, c->stream);
-    std::vector<double> h(2 * NC * (size_t)ns);
+    std::vector<double> h(NC * (size_t)ns);
     if (e == hipSuccess) {
-        launch_tri_rows(c->stream, tri_medium(G, lambda), dS, ns, dR, 1, kind, nullptr, 0, 0, 0, dout,
-                        dout + NC * (size_t)ns, ns, true);
+        const dim3 grid((ns + 63) / 64);
+        if (kind == 0)
+            hipLaunchKernelGGL((tri_hook_kernel<0>), grid, dim3(64), 0, c->stream,
+                               tri_medium(G, lambda), dS, ns, dR, dout);
+        else
+            hipLaunchKernelGGL((tri_hook_kernel<1>), grid, dim3(64), 0, c->stream,
+                               tri_medium(G, lambda), dS, ns, dR, dout);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(h.data(), dout, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream);
