@@ -49,7 +49,10 @@ struct ucy_ensemble {
     bool use_mlp = false;
     std::vector<double> tune_seconds;
     double gemm_bytes = 0;
-    int *h_done = nullptr;   // pinned host copy of the finished-instance count
+    int *h_done = nullptr;   // pinned host copy of the table's all_done
+    std::vector<double *> y0;    // per group: the initial state in the group's layout
+    double *stage = nullptr;     // one group's state in the caller's layout
+    char *ctl = nullptr;         // every group's control, kCtlBytes each
 };
 
 static int efail(ucy_ensemble *E, int code, const char *fmt, ...)
@@ -110,6 +113,9 @@ static void release(ucy_ensemble *E)
     if (E->h_done) (void)hipHostFree(E->h_done);
     E->h_done = nullptr;
     E->d_tab = nullptr;
+    E->y0.clear();
+    E->stage = nullptr;
+    E->ctl = nullptr;
     E->built = false;
 }
 
@@ -171,44 +177,18 @@ extern "C" int ucy_ensemble_add_group(ucy_ensemble *E, int np, const double *x, 
     return head;
 }
 
-// upload y0 (reference layout per instance) into the SoA state and reset control
+// the initial states, laid out on the device by the build, into the state; the
+// control back to the start
 static int load_initial(ucy_ensemble *E, double dt0)
 {
     ucy_ctx *c = E->ctx;
     for (size_t gi = 0; gi < E->hg.size(); gi++) {
-        const HostGroup &H = E->hg[gi];
         EnsGroup &G = E->tab.g[gi];
-        const int N = H.N;
-        std::vector<double> Y((size_t)7 * N * kEnsCols, 0.0);
-        for (int i = 0; i < H.ninst; i++)
-            for (int e = 0; e < N; e++)
-                for (int k = 0; k < 7; k++)
-                    Y[((size_t)k * N + e) * kEnsCols + i] = H.y0[((size_t)i * N + e) * 7 + k];
-        EHIP(hipMemcpyAsync(G.y, Y.data(), sizeof(double) * Y.size(), hipMemcpyHostToDevice, c->stream));
-        std::vector<double> hv(kEnsCols, dt0), zero(kEnsCols, 0.0);
-        std::vector<int> one(kEnsCols, 1), izero(kEnsCols, 0);
-        std::vector<long long> lzero(kEnsCols, 0);
-        EHIP(hipMemcpyAsync(G.h, hv.data(), sizeof(double) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.hnext, hv.data(), sizeof(double) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.time, zero.data(), sizeof(double) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.vmax, zero.data(), sizeof(double) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        std::vector<double> none(kEnsCols, -1.0);
-        EHIP(hipMemcpyAsync(G.t_event, none.data(), sizeof(double) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        std::vector<double> hz(5 * kEnsCols, 0.0);
-        EHIP(hipMemcpyAsync(G.hist, hz.data(), sizeof(double) * hz.size(), hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.errmax, zero.data(), sizeof(double) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        std::vector<double> zrep(kMaxRep * kEnsCols, 0.0);
-        EHIP(hipMemcpyAsync(G.vmax_rep, zrep.data(), sizeof(double) * zrep.size(), hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.errmax_rep, zrep.data(), sizeof(double) * zrep.size(), hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.need_rhs, one.data(), sizeof(int) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.accepted, izero.data(), sizeof(int) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.done, izero.data(), sizeof(int) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.status, izero.data(), sizeof(int) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.steps, lzero.data(), sizeof(long long) * kEnsCols, hipMemcpyHostToDevice, c->stream));
-        EHIP(hipMemcpyAsync(G.attempts, lzero.data(), sizeof(long long) * kEnsCols, hipMemcpyHostToDevice, c->stream));
+        EHIP(hipMemcpyAsync(G.y, E->y0[gi], sizeof(double) * 7 * (size_t)G.N * kEnsCols,
+                            hipMemcpyDeviceToDevice, c->stream));
     }
-    int z = 0;
-    EHIP(hipMemcpyAsync(E->tab.all_done, &z, sizeof(int), hipMemcpyHostToDevice, c->stream));
+    ens_launch_reset(c->stream, E->d_tab, E->tab, dt0);
+    EHIP(hipGetLastError());
     EHIP(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -274,6 +254,10 @@ extern "C" int ucy_ensemble_build(ucy_ensemble *E)
     T.ngroups = (int)E->hg.size();
     int eacc = 0, iacc = 0, total = 0;
     double bytes = 0;
+    size_t most = 0;
+    for (const HostGroup &H : E->hg) most = std::max(most, H.y0.size());
+    if (ealloc(E, &E->stage, most)) return UCY_ERR_HIP;
+    if (ealloc(E, &E->ctl, kCtlBytes * T.ngroups)) return UCY_ERR_HIP;
     for (int gi = 0; gi < T.ngroups; gi++) {
         const HostGroup &H = E->hg[gi];
         EnsGroup &G = T.g[gi];
@@ -405,20 +389,38 @@ extern "C" int ucy_ensemble_build(ucy_ensemble *E)
                 EHIP(hipMemcpyAsync(ds[k], hs[k]->data(), sizeof(double) * F, hipMemcpyHostToDevice, c->stream));
             EHIP(hipStreamSynchronize(c->stream));
         }
-        double **cv[] = {&G.time, &G.h, &G.hnext, &G.hdid, &G.errmax, &G.vmax, &G.t_event,
-                         &G.hstart};
-        for (double **v : cv)
-            if (ealloc(E, v, kEnsCols)) return UCY_ERR_HIP;
-        int **ci[] = {&G.need_rhs, &G.accepted, &G.done, &G.status};
-        for (int **v : ci)
-            if (ealloc(E, v, kEnsCols)) return UCY_ERR_HIP;
+        {
+            char *p = E->ctl + kCtlBytes * gi;
+            double **cv[] = {&G.time, &G.h, &G.hnext, &G.hdid, &G.errmax, &G.vmax, &G.t_event,
+                             &G.hstart};
+            for (double **v : cv) {
+                *v = (double *)p;
+                p += sizeof(double) * kEnsCols;
+            }
+            long long **cl[] = {&G.steps, &G.attempts};
+            for (long long **v : cl) {
+                *v = (long long *)p;
+                p += sizeof(long long) * kEnsCols;
+            }
+            int **ci[] = {&G.need_rhs, &G.accepted, &G.done, &G.status};
+            for (int **v : ci) {
+                *v = (int *)p;
+                p += sizeof(int) * kEnsCols;
+            }
+        }
         if (ealloc(E, &G.hist, 5 * kEnsCols)) return UCY_ERR_HIP;
         if (ealloc(E, &G.vmax_rep, kMaxRep * kEnsCols)) return UCY_ERR_HIP;
         if (ealloc(E, &G.errmax_rep, kMaxRep * kEnsCols)) return UCY_ERR_HIP;
         G.slog = nullptr;
         G.slog_cap = 0;
-        if (ealloc(E, &G.steps, kEnsCols)) return UCY_ERR_HIP;
-        if (ealloc(E, &G.attempts, kEnsCols)) return UCY_ERR_HIP;
+        // the initial state in the group's layout
+        double *y0 = nullptr;
+        if (ealloc(E, &y0, S7)) return UCY_ERR_HIP;
+        E->y0.push_back(y0);
+        EHIP(hipMemcpyAsync(E->stage, H.y0.data(), sizeof(double) * H.y0.size(),
+                            hipMemcpyHostToDevice, c->stream));
+        ens_launch_to_group(c->stream, E->stage, y0, G.N, G.ninst);
+        EHIP(hipGetLastError());
         T.blk_elem[gi] = eacc;
         eacc += (G.N + 3) / 4;
         T.blk_inst[gi] = iacc;
@@ -442,12 +444,12 @@ extern "C" int ucy_ensemble_build(ucy_ensemble *E)
     T.epsilon = 1e-6;
     T.max_step = 1.7976931348623157e308;
     T.max_attempts = 1;
-    if (ealloc(E, &T.all_done, 1)) return UCY_ERR_HIP;
+    if (ealloc(E, &T.all_done, 2)) return UCY_ERR_HIP;
     void *dt = nullptr;
     EHIP(hipMalloc(&dt, sizeof(EnsTable)));
     E->allocs.push_back(dt);
     E->d_tab = (EnsTable *)dt;
-    EHIP(hipHostMalloc((void **)&E->h_done, sizeof(int), hipHostMallocDefault));
+    EHIP(hipHostMalloc((void **)&E->h_done, 2 * sizeof(int), hipHostMallocDefault));
     E->gemm_bytes = bytes;
     // ---- tune the split-K tiling on the device: time the all-groups GEMM
     E->tune_seconds.clear();
@@ -464,33 +466,25 @@ extern "C" int ucy_ensemble_build(ucy_ensemble *E)
         hipEvent_t e0, e1;
         EHIP(hipEventCreate(&e0));
         EHIP(hipEventCreate(&e1));
-        // (split-bf16 variant, k-blocks per split); the binary64 GEMM has one
-        // variant
-        for (int ci = 0; ci < kGemmVariants * kDepths; ci++) {
-            const int kb = cands[ci % kDepths], v = ci / kDepths;
+        // one candidate: its seconds per launch (-1: not admissible) in t, and
+        // the choice so far
+        auto try_tiling = [&](int kb, int v, double &t) -> int {
+            t = -1.0;
             // binary64 has one variant; the LDS variants stage one V per
             // block and so serve families of one slice only
             if ((v > 0 && E->mode == 1) || (ens_gemm_variant_lds(v) && has_shared_families(T)) ||
-                (ens_gemm_variant_dma(v) && (E->mode != 3 || !kDmaVariantsOn))) {
-                E->tune_seconds.push_back(-1.0);
-                continue;
-            }
+                (ens_gemm_variant_dma(v) && (E->mode != 3 || !kDmaVariantsOn)))
+                return 0;
             set_split(T, kb, v);
-            bool ok = true;
             for (int gi = 0; gi < T.ngroups; gi++)
-                if (T.g[gi].ksplit > kMaxSplit) ok = false;
-            if (!ok) {
-                E->tune_seconds.push_back(-1.0);
-                continue;
-            }
+                if (T.g[gi].ksplit > kMaxSplit) return 0;
             if (upload_table(E)) return UCY_ERR_HIP;
             // 2 warm launches, 15 timed (single launches vary by ~10 %); a
             // candidate whose launch fails is not admissible
             for (int r = 0; r < 2; r++) ens_launch_gemm(c->stream, E->d_tab, T, 2);
             if (hipGetLastError() != hipSuccess) {
                 EHIP(hipStreamSynchronize(c->stream));
-                E->tune_seconds.push_back(-1.0);
-                continue;
+                return 0;
             }
             EHIP(hipEventRecord(e0, c->stream));
             for (int r = 0; r < 15; r++) ens_launch_gemm(c->stream, E->d_tab, T, 2);
@@ -499,8 +493,7 @@ extern "C" int ucy_ensemble_build(ucy_ensemble *E)
             EHIP(hipEventSynchronize(e1));
             float ms = 0;
             EHIP(hipEventElapsedTime(&ms, e0, e1));
-            const double t = 1e-3 * ms / 15;
-            E->tune_seconds.push_back(t);
+            t = 1e-3 * ms / 15;
             // the choice also charges the post-pass's read of the partial
             // products, one per split, at 4 TB/s (what the attempt measures:
             // a deeper split's extra partials cost the post kernels about
@@ -515,6 +508,14 @@ extern "C" int ucy_ensemble_build(ucy_ensemble *E)
                 best = kb;
                 best_v = v;
             }
+            return 0;
+        };
+        // (split-bf16 variant, k-blocks per split); the binary64 GEMM has one
+        // variant
+        for (int ci = 0; ci < kGemmVariants * kDepths; ci++) {
+            double t;
+            if (try_tiling(cands[ci % kDepths], ci / kDepths, t)) return UCY_ERR_HIP;
+            E->tune_seconds.push_back(t);
         }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
@@ -580,18 +581,21 @@ extern "C" int ucy_ensemble_run(ucy_ensemble *E, double t_end, int64_t max_attem
     if (upload_table(E)) return UCY_ERR_HIP;
     if (capture(E)) return UCY_ERR_HIP;
     // continue from the current state: re-arm every instance short of t_end
-    EHIP(hipMemsetAsync(E->tab.all_done, 0, sizeof(int), c->stream));
+    EHIP(hipMemsetAsync(E->tab.all_done, 0, 2 * sizeof(int), c->stream));
     ens_launch_rearm(c->stream, E->d_tab, E->tab);
     EHIP(hipGetLastError());
     int *h_done = E->h_done;   // allocated with the ensemble, freed by release()
-    EHIP(hipMemcpyAsync(h_done, E->tab.all_done, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    EHIP(hipMemcpyAsync(h_done, E->tab.all_done, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
     EHIP(hipStreamSynchronize(c->stream));
+    int64_t left = h_done[1];   // attempts after which every instance has used its own
     auto t0 = std::chrono::steady_clock::now();
     int batch = 8;
     int64_t replays = 0;
     for (; *h_done < E->tab.total_inst;) {
-        for (int i = 0; i < batch; i++) EHIP(hipGraphLaunch(E->graph, c->stream));
-        replays += batch;
+        const int64_t now = left > 0 ? std::min<int64_t>(batch, left) : batch;
+        for (int64_t i = 0; i < now; i++) EHIP(hipGraphLaunch(E->graph, c->stream));
+        replays += now;
+        left -= now;
         EHIP(hipMemcpyAsync(h_done, E->tab.all_done, sizeof(int), hipMemcpyDeviceToHost, c->stream));
         EHIP(hipStreamSynchronize(c->stream));
         if (*h_done >= E->tab.total_inst) break;
@@ -604,22 +608,21 @@ extern "C" int ucy_ensemble_run(ucy_ensemble *E, double t_end, int64_t max_attem
     if (stats) {
         memset(stats, 0, sizeof(*stats));
         stats->min_time = 1e300;
+        std::vector<char> ctl(kCtlBytes * E->tab.ngroups);
+        EHIP(hipMemcpy(ctl.data(), E->ctl, ctl.size(), hipMemcpyDeviceToHost));
         for (int gi = 0; gi < E->tab.ngroups; gi++) {
             const EnsGroup &G = E->tab.g[gi];
-            std::vector<double> tm(kEnsCols);
-            std::vector<long long> st(kEnsCols), at(kEnsCols);
-            std::vector<int> status(kEnsCols);
-            EHIP(hipMemcpy(tm.data(), G.time, sizeof(double) * kEnsCols, hipMemcpyDeviceToHost));
-            EHIP(hipMemcpy(st.data(), G.steps, sizeof(long long) * kEnsCols, hipMemcpyDeviceToHost));
-            EHIP(hipMemcpy(at.data(), G.attempts, sizeof(long long) * kEnsCols, hipMemcpyDeviceToHost));
-            EHIP(hipMemcpy(status.data(), G.status, sizeof(int) * kEnsCols, hipMemcpyDeviceToHost));
+            auto host = [&](auto *p) {
+                return (decltype(p))(ctl.data() + ((char *)p - E->ctl));
+            };
             for (int i = 0; i < G.ninst; i++) {
-                stats->inst_time_sum += tm[i];
-                stats->min_time = std::min(stats->min_time, tm[i]);
-                stats->max_time = std::max(stats->max_time, tm[i]);
-                stats->steps += st[i];
-                stats->attempts += at[i];
-                stats->n_failed += status[i] != 0;
+                const double t = host(G.time)[i];
+                stats->inst_time_sum += t;
+                stats->min_time = std::min(stats->min_time, t);
+                stats->max_time = std::max(stats->max_time, t);
+                stats->steps += host(G.steps)[i];
+                stats->attempts += host(G.attempts)[i];
+                stats->n_failed += host(G.status)[i] != 0;
             }
             stats->n_inst += G.ninst;
         }
@@ -749,32 +752,22 @@ extern "C" int ucy_ensemble_get_state(ucy_ensemble *E, int group, double *y, dou
     EHIP(hipSetDevice(E->ctx->device));
     EHIP(hipStreamSynchronize(E->ctx->stream));
     const EnsGroup &G = E->tab.g[group];
-    const HostGroup &H = E->hg[group];
     if (y) {
-        std::vector<double> Y((size_t)7 * G.N * kEnsCols);
-        EHIP(hipMemcpy(Y.data(), G.y, sizeof(double) * Y.size(), hipMemcpyDeviceToHost));
-        for (int i = 0; i < H.ninst; i++)
-            for (int e = 0; e < H.N; e++)
-                for (int k = 0; k < 7; k++)
-                    y[((size_t)i * H.N + e) * 7 + k] = Y[((size_t)k * G.N + e) * kEnsCols + i];
+        ens_launch_to_caller(E->ctx->stream, G.y, E->stage, G.N, G.ninst);
+        EHIP(hipGetLastError());
+        EHIP(hipMemcpyAsync(y, E->stage, sizeof(double) * 7 * (size_t)G.N * G.ninst,
+                            hipMemcpyDeviceToHost, E->ctx->stream));
     }
-    std::vector<double> tmp(kEnsCols);
-    std::vector<long long> lt(kEnsCols);
-    if (time) {
-        EHIP(hipMemcpy(tmp.data(), G.time, sizeof(double) * kEnsCols, hipMemcpyDeviceToHost));
-        std::copy(tmp.begin(), tmp.begin() + H.ninst, time);
-    }
-    if (dt_next) {
-        EHIP(hipMemcpy(tmp.data(), G.h, sizeof(double) * kEnsCols, hipMemcpyDeviceToHost));
-        std::copy(tmp.begin(), tmp.begin() + H.ninst, dt_next);
-    }
-    if (steps) {
-        EHIP(hipMemcpy(lt.data(), G.steps, sizeof(long long) * kEnsCols, hipMemcpyDeviceToHost));
-        for (int i = 0; i < H.ninst; i++) steps[i] = lt[i];
-    }
-    if (attempts) {
-        EHIP(hipMemcpy(lt.data(), G.attempts, sizeof(long long) * kEnsCols, hipMemcpyDeviceToHost));
-        for (int i = 0; i < H.ninst; i++) attempts[i] = lt[i];
+    std::vector<char> ctl(kCtlBytes);
+    char *base = E->ctl + kCtlBytes * group;
+    EHIP(hipMemcpyAsync(ctl.data(), base, kCtlBytes, hipMemcpyDeviceToHost, E->ctx->stream));
+    EHIP(hipStreamSynchronize(E->ctx->stream));
+    auto host = [&](auto *p) { return (decltype(p))(ctl.data() + ((char *)p - base)); };
+    for (int i = 0; i < G.ninst; i++) {
+        if (time) time[i] = host(G.time)[i];
+        if (dt_next) dt_next[i] = host(G.h)[i];
+        if (steps) steps[i] = host(G.steps)[i];
+        if (attempts) attempts[i] = host(G.attempts)[i];
     }
     return UCY_OK;
 }
@@ -858,7 +851,7 @@ extern "C" int ucy_ensemble_time_phases(ucy_ensemble *E, int attempts, double *p
     E->tab.mlp = E->use_mlp ? E->d_mlp : nullptr;
     E->tab.mlp_norm = E->mlp_norm;
     if (upload_table(E)) return UCY_ERR_HIP;
-    EHIP(hipMemsetAsync(E->tab.all_done, 0, sizeof(int), c->stream));
+    EHIP(hipMemsetAsync(E->tab.all_done, 0, 2 * sizeof(int), c->stream));
     ens_launch_rearm(c->stream, E->d_tab, E->tab);
     EHIP(hipGetLastError());
     hipEvent_t ev[UCY_ENS_PHASES + 1];

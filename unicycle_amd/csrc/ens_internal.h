@@ -97,7 +97,7 @@ struct EnsTable {
     double event_vmax;              // slip-velocity threshold of an event (m/s)
     const float *mlp;               // step-size proposal parameters (null: classic control)
     MlpNorm mlp_norm;
-    int *all_done;                  // count of finished instances
+    int *all_done;                  // [2] finished instances; most attempts left to one
     int total_inst;
 };
 
@@ -122,7 +122,16 @@ int ens_gemm_variant_lds(int variant);
 int ens_gemm_variant_dma(int variant);
 int ens_gemm_variant_kshare(int variant);
 
+// a group's per-instance control in one block, so that the host reads it in one
+// copy: eight binary64 arrays (time, h, hnext, hdid, errmax, vmax, t_event,
+// hstart), steps and attempts, then need_rhs, accepted, done and status
+constexpr size_t kCtlBytes = (8 * 8 + 2 * 8 + 4 * 4) * kEnsCols;
+
 // launchers (k_ensemble.hip)
+// states between the caller's layout and a group's
+void ens_launch_to_group(hipStream_t st, double *caller, double *group, int N, int ninst);
+void ens_launch_to_caller(hipStream_t st, double *group, double *caller, int N, int ninst);
+void ens_launch_reset(hipStream_t st, const EnsTable *dtab, const EnsTable &h, double dt0);
 void ens_launch_split_K(hipStream_t st, const double *K, int m, int n, int mp, int np, uint16_t *tiles,
                         double *rscale);
 void ens_launch_split3_K(hipStream_t st, const double *K, int m, int n, int mp, int np,

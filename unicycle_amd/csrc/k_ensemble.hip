@@ -1916,7 +1916,93 @@ __global__ void ens_rearm_kernel(EnsTable *tab)
                        G.attempts[inst] < tab->max_attempts &&
                        !(tab->stop_at_event && G.t_event[inst] >= 0.0));
     G.done[inst] = done;
-    if (done) atomicAdd(tab->all_done, 1);
+    if (done) {
+        atomicAdd(tab->all_done, 1);
+    } else {
+        // each attempt of the ensemble is one of every unfinished instance: the
+        // largest number left bounds the call's attempts
+        const long long left = tab->max_attempts - G.attempts[inst];
+        atomicMax(tab->all_done + 1, (int)(left < (1 << 30) ? left : 1 << 30));
+    }
+}
+
+// A group's state between the caller's layout (instance, element, component)
+// and the group's (component, element, instance), through LDS: 8 elements of 64
+// instances per block, read in runs of 448 bytes and written in runs of 512, or
+// the other way round.  The host's loops over 64 instances each of 1024 to 8192
+// patches (55 MB) and their copies took 130 ms for a reset and a read-back; this
+// and the copy of the states to the caller take 5 ms, nearly all of it the copy.
+constexpr int kTileElems = 8, kTileRow = 7 * kTileElems;
+template <bool TO_GROUP>
+__global__ void __launch_bounds__(256)
+ens_layout_kernel(double *__restrict__ caller, double *__restrict__ group, int N, int ninst)
+{
+    __shared__ double tile[kEnsCols][kTileRow + 1];
+    const int e0 = blockIdx.x * kTileElems, ne = min(kTileElems, N - e0), row = 7 * ne;
+    auto caller_side = [&]() {
+        for (int i = threadIdx.x; i < ninst * row; i += 256) {
+            const int inst = i / row, c = i - inst * row;
+            double &x = caller[((size_t)inst * N + e0) * 7 + c];
+            if (TO_GROUP) tile[inst][c] = x;
+            else x = tile[inst][c];
+        }
+    };
+    auto group_side = [&]() {
+        const int inst = threadIdx.x & 63;
+        for (int j = threadIdx.x >> 6; j < row; j += 4) {
+            const int k = j / ne, e = j - k * ne;
+            double &x = group[((size_t)k * N + e0 + e) * kEnsCols + inst];
+            if (TO_GROUP) x = inst < ninst ? tile[inst][7 * e + k] : 0.0;
+            else if (inst < ninst) tile[inst][7 * e + k] = x;
+        }
+    };
+    if (TO_GROUP) caller_side();
+    else group_side();
+    __syncthreads();
+    if (TO_GROUP) group_side();
+    else caller_side();
+}
+
+void ens_launch_to_group(hipStream_t st, double *caller, double *group, int N, int ninst)
+{
+    hipLaunchKernelGGL((ens_layout_kernel<true>), dim3((N + kTileElems - 1) / kTileElems),
+                       dim3(256), 0, st, caller, group, N, ninst);
+}
+void ens_launch_to_caller(hipStream_t st, double *group, double *caller, int N, int ninst)
+{
+    hipLaunchKernelGGL((ens_layout_kernel<false>), dim3((N + kTileElems - 1) / kTileElems),
+                       dim3(256), 0, st, caller, group, N, ninst);
+}
+
+// the step control of every instance back to the start of a run
+__global__ void ens_reset_kernel(EnsTable *tab, double dt0)
+{
+    const EnsGroup &G = tab->g[blockIdx.x];
+    const int inst = threadIdx.x;
+    G.h[inst] = dt0;
+    G.hnext[inst] = dt0;
+    G.time[inst] = 0.0;
+    G.vmax[inst] = 0.0;
+    G.t_event[inst] = -1.0;
+    G.errmax[inst] = 0.0;
+    for (int k = 0; k < 5; k++) G.hist[k * kEnsCols + inst] = 0.0;
+    for (int r = 0; r < kMaxRep; r++) {
+        G.vmax_rep[r * kEnsCols + inst] = 0.0;
+        G.errmax_rep[r * kEnsCols + inst] = 0.0;
+    }
+    G.need_rhs[inst] = 1;
+    G.accepted[inst] = 0;
+    G.done[inst] = 0;
+    G.status[inst] = 0;
+    G.steps[inst] = 0;
+    G.attempts[inst] = 0;
+    if (blockIdx.x == 0 && inst < 2) tab->all_done[inst] = 0;
+}
+
+void ens_launch_reset(hipStream_t st, const EnsTable *dtab, const EnsTable &h, double dt0)
+{
+    hipLaunchKernelGGL(ens_reset_kernel, dim3(h.ngroups), dim3(kEnsCols), 0, st,
+                       const_cast<EnsTable *>(dtab), dt0);
 }
 
 void ens_launch_rearm(hipStream_t st, const EnsTable *dtab, const EnsTable &h)
