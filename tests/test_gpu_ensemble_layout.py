@@ -3,7 +3,8 @@ run issues, and the shallow k-splits that small ensembles take."""
 import numpy as np
 import pytest
 
-from unicycle_amd import PREC_F64, PREC_SPLIT_BF16, configs
+import orc
+from unicycle_amd import PREC_BF16_I8, PREC_F64, PREC_SPLIT_BF16, configs
 from unicycle_amd.ensemble import Ensemble
 
 pytestmark = pytest.mark.gpu
@@ -61,5 +62,26 @@ def test_two_groups_and_a_continued_run(engine_factory):
     assert replays == whole.replays == 50
     for g in range(2):
         assert np.array_equal(ens.state(g)[0], end[g])
+    ens.close()
+    eng.close()
+
+
+@pytest.mark.parametrize("nx,nz", [(17, 9), (24, 12), (13, 3)])
+@pytest.mark.parametrize("precision,bound", [(PREC_F64, 1e-14), (PREC_BF16_I8, 2.0 ** -13)])
+def test_shallow_splits(engine_factory, nx, nz, precision, bound):
+    """Every depth from 2 k-blocks per split up, remainders included, against
+    binary64 (the bounds of the ensemble matvec)."""
+    eng = engine_factory()
+    ens, y0s = _ensemble(eng, precision, [(nx, nz)], 9)
+    m = y0s[0][0]
+    K = orc.buildG(orc.Mesh(m.lambda_, m.mu, rect=m.geometry()), nthreads=8)
+    V = np.random.default_rng(1).standard_normal((2 * m.n, 9))
+    want, scale = K @ V, np.abs(K) @ np.abs(V)
+    nkb = (2 * m.n + 15) // 16
+    for kb in [ens.tuning()[0], 2, 3, 4, 6, 8, 12, 16, 24]:
+        if (nkb + kb - 1) // kb > 16:
+            continue
+        ens.set_tiling(kb, 0 if precision == PREC_F64 else 5)
+        assert np.all(np.abs(ens.matvec(0, V) - want) <= bound * scale), kb
     ens.close()
     eng.close()

@@ -517,6 +517,19 @@ extern "C" int ucy_ensemble_build(ucy_ensemble *E)
             if (try_tiling(cands[ci % kDepths], ci / kDepths, t)) return UCY_ERR_HIP;
             E->tune_seconds.push_back(t);
         }
+        // Small ensembles: where the least depth of the table leaves CUs without
+        // a block, a wave's chain over its k-blocks is the launch.  Shallower
+        // splits (not in the table) shorten it and fill the chip: the binary64
+        // launch of 37 instances of 288 and 153 patches, 9 blocks at 32 k-blocks
+        // per split, goes from 54 to 12 us, the post-passes' read of up to 16
+        // partial products from 6 to 13 us.
+        set_split(T, cands[0], 0);
+        if ((E->mode == 1 ? T.blk_gemm64[T.nfam] : T.blk_gemm[T.nfam]) < 256)
+            for (int kb : {2, 3, 4, 6, 8, 12, 16, 24})
+                for (int v = 0; v < kGemmVariants; v++) {
+                    double t;
+                    if (try_tiling(kb, v, t)) return UCY_ERR_HIP;
+                }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         if (!best) return efail(E, UCY_ERR_STATE, "no admissible GEMM tiling");
