@@ -2,13 +2,15 @@
 // columns of K and the per-kernel hooks of strainvolume.f90:4671-4799.
 //
 // One lane per (receiver, source volume) pair computes the stress of all six
-// unit eigenstrains at once: the 8-corner sum of the displacement
-// J-integrals (sv_jint.h) differentiated in forward mode with respect to the
-// observation point, then strain, rotation, eigenstrain removal inside the
-// volume and Hooke (strainvolume.f90:1042-1138), then the traction projection
-// for patch receivers or the volume-frame stress for volume receivers.
+// unit eigenstrains at once: the 8-corner sums of the displacement gradients
+// (sv_dev.h; on the planes of a volume's faces the J-integrals of sv_jint.h
+// differentiated in forward mode with respect to the observation point), then
+// strain, rotation, eigenstrain removal inside the volume and Hooke
+// (strainvolume.f90:1042-1138), then the traction projection for patch receivers
+// or the volume-frame stress for volume receivers.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <cmath>
 #include <vector>
 #include "ucy_ext.h"
 #include "ucy_ctx.h"
@@ -121,6 +123,7 @@ VD_FN VV sv_acoth(const VV &X)
 }  // namespace ucy
 
 #include "sv_jint.h"
+#include "sv_dev.h"
 
 namespace svj {
 template <>
@@ -144,24 +147,34 @@ struct SvSource {
     double q[3], L, T, W, strike;
 };
 
+// the receiver's position in the source's frame (strainvolume.f90:1074-1077); one
+// place, so that both kernels below see the same bits
+__device__ __forceinline__ void sv_frame(const Receiver &R, const SvSource &S, double ct, double st,
+                                         double &x1p, double &x2p)
+{
+    x1p = (R.xc[0] - S.q[0]) * ct + (R.xc[1] - S.q[1]) * st;
+    x2p = -(R.xc[0] - S.q[0]) * st + (R.xc[1] - S.q[1]) * ct;
+}
+
+// On the plane of one of the volume's vertical faces, where terms of the formulas
+// are 0/0 (squares: the quotients are of squared distances)
+__device__ __forceinline__ bool sv_on_plane(const SvSource &S, double x1p, double x2p)
+{
+    const double a0 = x1p - S.L, b0 = x2p - S.T / 2.0, b1 = x2p + S.T / 2.0;
+    return a0 * a0 == 0.0 || x1p * x1p == 0.0 || b0 * b0 == 0.0 || b1 * b1 == 0.0;
+}
+
+// The six stress columns to rows of K and/or the hooks' layout.
 // KIND 0: traction rows (3) of patch receivers; 1: volume-frame stress rows (6)
 template <int KIND>
-__global__ void __launch_bounds__(128)
-sv_rows_kernel(double G, double nu, const SvSource *__restrict__ src, int ns,
-               const Receiver *__restrict__ rcv, double *__restrict__ K, int64_t ldk, int64_t row0,
-               int64_t col0, double *out, int out_stride)
+__device__ __forceinline__ void sv_store(const Receiver &R, const double st[6][6], int s, int r,
+                                         double *__restrict__ K, int64_t ldk, int64_t row0,
+                                         int64_t col0, double *out, int out_stride)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    const int r = blockIdx.y;
-    if (s >= ns) return;
-    const Receiver R = rcv[r];
-    const SvSource S = src[s];
-    double st[6][6];
-    svj::stress6<VD, SeedVD, true>(R.xc[0], R.xc[1], R.xc[2], S.q[0], S.q[1], S.q[2], S.L, S.T,
-                                   S.W, S.strike, G, nu, SeedVD(), st);
     constexpr int NC = KIND == 0 ? 3 : 6;
     double o[6][NC];
     const double *sv = R.sv, *dv = R.dv, *nv = R.nv;
+#pragma unroll
     for (int e = 0; e < 6; e++) {
         const double *S6 = st[e];
         if constexpr (KIND == 0) {  // strainvolume.f90:4699-4707
@@ -203,6 +216,58 @@ sv_rows_kernel(double G, double nu, const SvSource *__restrict__ src, int ns,
             for (int c = 0; c < NC; c++) out[(int64_t)(e * NC + c) * out_stride + s] = o[e][c];
 }
 
+// Every pair off the faces' planes.  Bound by the issue of vector instructions,
+// some 15 thousand per wave of pairs (four laps of two corners), at 1 wave per
+// SIMD; the columns of K are 8 % of the time at 7 TB/s.  594 volumes on 234
+// patches and on themselves: 78 + 162 us; the formula text differentiated in
+// forward mode for every pair took 1.19 + 2.67 ms.
+template <int KIND>
+__global__ void __launch_bounds__(64)
+sv_sums_kernel(SvMedium M, double G, double nu, double lambda, const SvSource *__restrict__ src,
+               int ns, const Receiver *__restrict__ rcv, double *__restrict__ K, int64_t ldk,
+               int64_t row0, int64_t col0, double *out, int out_stride)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    const int r = blockIdx.y;
+    if (s >= ns) return;
+    const Receiver &R = rcv[r];
+    const SvSource S = src[s];
+    const double ct = cos(S.strike), st = sin(S.strike);
+    double x1p, x2p;
+    sv_frame(R, S, ct, st, x1p, x2p);
+    if (sv_on_plane(S, x1p, x2p)) return;   // sv_planes_kernel's
+    SvSums A;
+    sv_sums(M, A, x1p, x2p, R.xc[2], S.q[2], S.L, S.T, S.W);
+    const double inside = svj::sv_s(x1p / S.L) * svj::sv_omega(x2p / S.T)
+                          * svj::sv_s((R.xc[2] - S.q[2]) / S.W);
+    double sig[6][6];
+    sv_stresses(A, G, nu, lambda, ct, st, inside, sig);
+    sv_store<KIND>(R, sig, s, r, K, ldk, row0, col0, out, out_stride);
+}
+
+// The pairs on a face's plane (or, with `all`, every pair: nu = 1/2, where lambda
+// is infinite): the formula text as it stands, with its 0/0.  Without such a pair
+// a launch reads the positions and ends, 5 + 9 us beside the above.
+template <int KIND>
+__global__ void __launch_bounds__(128)
+sv_planes_kernel(double G, double nu, bool all, const SvSource *__restrict__ src, int ns,
+                 const Receiver *__restrict__ rcv, double *__restrict__ K, int64_t ldk,
+                 int64_t row0, int64_t col0, double *out, int out_stride)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    const int r = blockIdx.y;
+    if (s >= ns) return;
+    const Receiver R = rcv[r];
+    const SvSource S = src[s];
+    double x1p, x2p;
+    sv_frame(R, S, cos(S.strike), sin(S.strike), x1p, x2p);
+    if (!all && !sv_on_plane(S, x1p, x2p)) return;
+    double st[6][6];
+    svj::stress6<VD, SeedVD, true>(R.xc[0], R.xc[1], R.xc[2], S.q[0], S.q[1], S.q[2], S.L, S.T,
+                                   S.W, S.strike, G, nu, SeedVD(), st);
+    sv_store<KIND>(R, st, s, r, K, ldk, row0, col0, out, out_stride);
+}
+
 struct SeedVV {
     __host__ __device__ VV operator()(double v, int) const { return VV(v); }
 };
@@ -236,13 +301,24 @@ static void launch_sv_rows(hipStream_t st, double G, double nu, const SvSource *
                            int64_t row0, int64_t col0, double *out, int stride)
 {
     if (ns <= 0 || nr <= 0) return;
-    const dim3 grid((ns + 127) / 128, nr);
+    const double lambda = G * 2.0 * nu / (1.0 - 2.0 * nu);
+    const bool all = !std::isfinite(lambda);
+    const SvMedium M = sv_medium(nu);
+    const dim3 sums((ns + 63) / 64, nr), planes((ns + 127) / 128, nr);
+    if (!all) {
+        if (kind == 0)
+            hipLaunchKernelGGL(sv_sums_kernel<0>, sums, dim3(64), 0, st, M, G, nu, lambda, src, ns,
+                               rcv, K, ldk, row0, col0, out, stride);
+        else
+            hipLaunchKernelGGL(sv_sums_kernel<1>, sums, dim3(64), 0, st, M, G, nu, lambda, src, ns,
+                               rcv, K, ldk, row0, col0, out, stride);
+    }
     if (kind == 0)
-        hipLaunchKernelGGL(sv_rows_kernel<0>, grid, dim3(128), 0, st, G, nu, src, ns, rcv, K, ldk,
-                           row0, col0, out, stride);
+        hipLaunchKernelGGL(sv_planes_kernel<0>, planes, dim3(128), 0, st, G, nu, all, src, ns, rcv,
+                           K, ldk, row0, col0, out, stride);
     else
-        hipLaunchKernelGGL(sv_rows_kernel<1>, grid, dim3(128), 0, st, G, nu, src, ns, rcv, K, ldk,
-                           row0, col0, out, stride);
+        hipLaunchKernelGGL(sv_planes_kernel<1>, planes, dim3(128), 0, st, G, nu, all, src, ns, rcv,
+                           K, ldk, row0, col0, out, stride);
 }
 
 // strainvolume.f90:1059-1072 (STOP in the reference)
