@@ -673,15 +673,22 @@ extern "C" int ucy_build_kernel(ucy_ctx *c, int precision)
         if (rc) return rc;
     }
     free_work(c);
-    if (c->K) HIPCHK(hipFree(c->K));
-    c->K = nullptr;
+    // A kernel of the same shape is written over: mapping and unmapping 137 MB
+    // took 0.2 ms of an assembly of 0.57 ms, at times 3 ms.  What else reads it,
+    // on any stream, has ended then, as it had when hipFree returned.
+    if (c->K && (c->m != m || c->n != n)) {
+        HIPCHK(hipFree(c->K));
+        c->K = nullptr;
+    } else if (c->K) {
+        HIPCHK(hipDeviceSynchronize());
+    }
     if (c->Kp) HIPCHK(hipFree(c->Kp));
     c->Kp = nullptr;
     if (c->Krs) HIPCHK(hipFree(c->Krs));
     c->Krs = nullptr;
     c->kprec = UCY_PREC_F64;
     if (n % 2) return fail(c, UCY_ERR_STATE, "odd column count");
-    HIPCHK(hipMalloc((void **)&c->K, (size_t)(m * n) * sizeof(double)));
+    if (!c->K) HIPCHK(hipMalloc((void **)&c->K, (size_t)(m * n) * sizeof(double)));
     c->m = m;
     c->n = n;
     c->nl = ap ? nap : ps ? nps : n;
@@ -790,8 +797,10 @@ extern "C" int ucy_build_kernel(ucy_ctx *c, int precision)
         return UCY_OK;
     }
     element_frames(c, R);
-    Receiver *d_R = nullptr;
-    HIPCHK(hipMalloc((void **)&d_R, sizeof(Receiver) * ne));
+    // receivers and rectangle sources in the context's scratch
+    const size_t rb = (sizeof(Receiver) * ne + 255) / 256 * 256;
+    if (ensure_buf(c, c->hook, rb + sizeof(OkadaSource) * c->nrect)) return UCY_ERR_HIP;
+    Receiver *d_R = (Receiver *)c->hook.p;
     HIPCHK(hipMemcpyAsync(d_R, R.data(), sizeof(Receiver) * ne, hipMemcpyHostToDevice, c->stream));
     int rc = 0;
     using clk = std::chrono::steady_clock;
@@ -806,8 +815,7 @@ extern "C" int ucy_build_kernel(ucy_ctx *c, int precision)
         std::vector<OkadaSource> S(c->nrect);
         for (int i = 0; i < c->nrect; i++)
             S[i] = make_source(&c->rx[3 * i], c->rL[i], c->rW[i], c->rstrike[i], c->rdip[i]);
-        OkadaSource *d_S = nullptr;
-        HIPCHK(hipMalloc((void **)&d_S, sizeof(OkadaSource) * c->nrect));
+        OkadaSource *d_S = (OkadaSource *)((char *)c->hook.p + rb);
         HIPCHK(hipMemcpyAsync(d_S, S.data(), sizeof(OkadaSource) * c->nrect,
                               hipMemcpyHostToDevice, c->stream));
         const OkadaMedium M = make_medium(c->mu, c->lambda);
@@ -823,7 +831,6 @@ extern "C" int ucy_build_kernel(ucy_ctx *c, int precision)
         }
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(c->stream));
-        HIPCHK(hipFree(d_S));
     }
     c->build_seconds[0] = since(t0);
     t0 = clk::now();
@@ -837,10 +844,10 @@ extern "C" int ucy_build_kernel(ucy_ctx *c, int precision)
     if (!rc && c->nvol)
         rc = ext_build_volume_columns(c->stream, c->mu, c->lambda, c->nvol, c->vx.data(),
                                       c->vL.data(), c->vT.data(), c->vW.data(),
-                                      c->vstrike.data(), d_R, np, c->K, n, 2 * (int64_t)np, c->err);
+                                      c->vstrike.data(), R.data(), d_R, np, c->K, n,
+                                      2 * (int64_t)np, c->err);
     HIPCHK(hipStreamSynchronize(c->stream));
     c->build_seconds[2] = since(t0);
-    HIPCHK(hipFree(d_R));
     if (!rc && precision != UCY_PREC_F64) {
         // the split pairs of K (4 bytes per entry) beside the binary64 K
         HIPCHK(hipMalloc((void **)&c->Kp, (size_t)(m * n) * sizeof(uint32_t)));

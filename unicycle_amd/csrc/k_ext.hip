@@ -329,8 +329,8 @@ static bool sv_bad(double nu, double x3, double q3)
 
 int ext_build_volume_columns(hipStream_t st, double G, double lambda, int nvol, const double *x,
                              const double *L, const double *T, const double *W,
-                             const double *strike, const Receiver *d_R, int np, double *K,
-                             int64_t ldk, int64_t col0, std::string &msg)
+                             const double *strike, const Receiver *R, const Receiver *d_R, int np,
+                             double *K, int64_t ldk, int64_t col0, std::string &msg)
 {
     // computeTractionKernels/StressKernelsVerticalStrainVolume: nu from lambda
     const double nu = lambda / (lambda + G) / 2.0;
@@ -342,15 +342,13 @@ int ext_build_volume_columns(hipStream_t st, double G, double lambda, int nvol, 
             return UCY_ERR_GEOMETRY;
         }
     }
-    std::vector<Receiver> R(np + nvol);
-    hipError_t e = hipMemcpy(R.data(), d_R, sizeof(Receiver) * (np + nvol), hipMemcpyDeviceToHost);
-    for (int i = 0; e == hipSuccess && i < np + nvol; i++)
+    for (int i = 0; i < np + nvol; i++)
         if (R[i].xc[2] < 0.0) {
             msg = "strain volume: observation depth must be positive";
             return UCY_ERR_GEOMETRY;
         }
     SvSource *dS = nullptr;
-    if (e == hipSuccess) e = hipMalloc((void **)&dS, sizeof(SvSource) * nvol);
+    hipError_t e = hipMalloc((void **)&dS, sizeof(SvSource) * nvol);
     if (e == hipSuccess) e = hipMemcpyAsync(dS, S.data(), sizeof(SvSource) * nvol, hipMemcpyHostToDevice, st);
     for (int r0 = 0; r0 < np && e == hipSuccess; r0 += 65535)
         launch_sv_rows(st, G, nu, dS, nvol, d_R + r0, std::min(65535, np - r0), 0, K, ldk,
