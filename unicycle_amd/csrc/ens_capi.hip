@@ -522,7 +522,7 @@ extern "C" int ucy_ensemble_build(ucy_ensemble *E)
         // splits (not in the table) shorten it and fill the chip: the binary64
         // launch of 37 instances of 288 and 153 patches, 9 blocks at 32 k-blocks
         // per split, goes from 54 to 12 us, the post-passes' read of up to 16
-        // partial products from 6 to 13 us.
+        // partial products from 6 to 8 us.
         set_split(T, cands[0], 0);
         if ((E->mode == 1 ? T.blk_gemm64[T.nfam] : T.blk_gemm[T.nfam]) < 256)
             for (int kb : {2, 3, 4, 6, 8, 12, 16, 24})
