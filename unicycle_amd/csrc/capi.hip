@@ -107,6 +107,7 @@ OkadaSource make_source(const double *x, double L, double W, double strike, doub
     S.sdsd = sd * sd;
     S.cdcd = cd * cd;
     S.sdcd = sd * cd;
+    S.icd = 1.0 / cd;
     return S;
 }
 

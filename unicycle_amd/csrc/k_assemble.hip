@@ -44,8 +44,13 @@ __device__ __forceinline__ void proj_volume(const Receiver &R, const double S[6]
     o[5] = -c1 * dv[0] - c2 * dv[1] - c3 * dv[2];
 }
 
+// Bound by binary64 arithmetic and its latencies: some 11 thousand instructions
+// per wave of pairs.  Two waves per SIMD (28 registers to scratch) hide more than
+// they cost: 2048 sources on themselves take 0.85 ms, at one wave (276 registers)
+// 0.94, and with divisions in place of the corrected reciprocals of okada_dev.h
+// 1.09 and 1.30.
 template <int KIND>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 2)
 okada_rows_kernel(OkadaMedium M, const OkadaSource *__restrict__ src, int ns,
                   const Receiver *__restrict__ rcv, double *__restrict__ K, int64_t ldk,
                   int64_t row0, int64_t col0, double *s_out, double *d_out, int out_stride)

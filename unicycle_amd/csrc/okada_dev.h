@@ -24,6 +24,7 @@ struct OkadaSource {
     double csst, ssst;      // cos/sin of strike
     double sd, cd;          // DCCON0 sin/cos of the binary32 dip in degrees
     double sdsd, cdcd, sdcd;
+    double icd;             // 1/cd
     float depth, al2, aw1;  // SNGL(q3), SNGL(L), -SNGL(W)
     float pad;
 };
@@ -33,7 +34,37 @@ struct OkadaMedium {
     double G, lambda;
 };
 
+// A divisor with its reciprocal to a few ulp.  over() is the quotient rounded as by
+// division, but for ties to within the reciprocal's squared error: an estimate and
+// one correction by its exact residual (Markstein 1990), 3 instructions where a
+// division takes 11.  The divisors here are lengths and their products: not zero
+// (the singular edges have left before) and far from the ends of the range.
+struct Divisor {
+    double d, inv;
+};
+__device__ __forceinline__ double over(double n, const Divisor &D)
+{
+    const double q = n * D.inv;
+    return fma(fma(-D.d, q, n), D.inv, q);
+}
+__device__ __forceinline__ Divisor divisor(double d)
+{
+    double y = __builtin_amdgcn_rcp(d);
+    y = fma(fma(-d, y, 1.0), y, y);
+    return {d, fma(fma(-d, y, 1.0), y, y)};
+}
+// sqrt(x) likewise, with its reciprocal; x > 0
+__device__ __forceinline__ Divisor root(double x)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+    y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+    const double s = x * y;
+    return {fma(fma(-s, s, x), 0.5 * y, s), y};
+}
+
 struct DcGeo {
+    Divisor R, R2, R3, R5;   // r and its powers as divisors
     double xi2, et2, q2, r, r2, r3, r5, y, d, tt, alx, ale, x11, y11, x32, y32;
     double ey, ez, fy, fz, gy, gz, hy, hz;
 };
@@ -49,10 +80,19 @@ __device__ __forceinline__ void dc_geo(DcGeo &g, double &xi, double &et, double 
     g.et2 = et * et;
     g.q2 = q * q;
     g.r2 = g.xi2 + g.et2 + g.q2;
-    g.r = sqrt(g.r2);
-    if (g.r == 0.0) return;  // the reference keeps the previous corner's terms
+    if (g.r2 == 0.0) {  // the reference keeps the previous corner's terms
+        g.r = 0.0;
+        g.R = g.R2 = {0.0, __builtin_inf()};
+        return;
+    }
+    g.R = root(g.r2);
+    g.r = g.R.d;
     g.r3 = g.r * g.r2;
     g.r5 = g.r3 * g.r2;
+    const double i2 = g.R.inv * g.R.inv, i3 = i2 * g.R.inv;
+    g.R2 = {g.r2, i2};
+    g.R3 = {g.r3, i3};
+    g.R5 = {g.r5, i3 * i2};
     g.y = et * cd + q * sd;
     g.d = et * sd - q * cd;
     g.tt = (q == 0.0) ? 0.0 : atan(xi * et / (q * g.r));
@@ -63,8 +103,8 @@ __device__ __forceinline__ void dc_geo(DcGeo &g, double &xi, double &et, double 
     } else {
         double rxi = g.r + xi;
         g.alx = log(rxi);
-        g.x11 = 1.0 / (g.r * rxi);
-        g.x32 = (g.r + rxi) * g.x11 * g.x11 / g.r;
+        g.x11 = over(1.0, divisor(g.r * rxi));
+        g.x32 = over((g.r + rxi) * g.x11 * g.x11, g.R);
     }
     if (ket == 1) {
         g.ale = -log(g.r - et);
@@ -73,13 +113,13 @@ __device__ __forceinline__ void dc_geo(DcGeo &g, double &xi, double &et, double 
     } else {
         double ret = g.r + et;
         g.ale = log(ret);
-        g.y11 = 1.0 / (g.r * ret);
-        g.y32 = (g.r + ret) * g.y11 * g.y11 / g.r;
+        g.y11 = over(1.0, divisor(g.r * ret));
+        g.y32 = over((g.r + ret) * g.y11 * g.y11, g.R);
     }
-    g.ey = sd / g.r - g.y * q / g.r3;
-    g.ez = cd / g.r + g.d * q / g.r3;
-    g.fy = g.d / g.r3 + g.xi2 * g.y32 * sd;
-    g.fz = g.y / g.r3 + g.xi2 * g.y32 * cd;
+    g.ey = over(sd, g.R) - over(g.y * q, g.R3);
+    g.ez = over(cd, g.R) + over(g.d * q, g.R3);
+    g.fy = over(g.d, g.R3) + g.xi2 * g.y32 * sd;
+    g.fz = over(g.y, g.R3) + g.xi2 * g.y32 * cd;
     g.gy = 2.0 * g.x11 * sd - g.y * q * g.x32;
     g.gz = 2.0 * g.x11 * cd + g.d * q * g.x32;
     g.hy = g.d * q * g.x32 + xi * q * g.y32 * sd;
@@ -95,23 +135,23 @@ __device__ __forceinline__ void dc_ua2(const OkadaMedium &M, const OkadaSource &
     const double a1 = M.alp1, a2 = M.alp2, sd = S.sd, cd = S.cd;
     const double xy = xi * g.y11, qx = q * g.x11, qy = q * g.y11;
     us[0] = c * (g.tt / 2.0 + a2 * xi * qy);
-    us[1] = c * (a2 * q / g.r);
+    us[1] = c * (over(a2 * q, g.R));
     us[2] = c * (a1 * g.ale - a2 * q * qy);
     us[3] = c * (-a1 * qy - a2 * g.xi2 * q * g.y32);
-    us[4] = c * (-a2 * xi * q / g.r3);
+    us[4] = c * (over(-a2 * xi * q, g.R3));
     us[5] = c * (a1 * xy + a2 * xi * g.q2 * g.y32);
     us[6] = c * (a1 * xy * sd + a2 * xi * g.fy + g.d / 2.0 * g.x11);
     us[7] = c * (a2 * g.ey);
-    us[8] = c * (a1 * (cd / g.r + qy * sd) - a2 * q * g.fy);
+    us[8] = c * (a1 * (over(cd, g.R) + qy * sd) - a2 * q * g.fy);
     us[9] = c * (a1 * xy * cd + a2 * xi * g.fz + g.y / 2.0 * g.x11);
     us[10] = c * (a2 * g.ez);
-    us[11] = c * (-a1 * (sd / g.r - qy * cd) - a2 * q * g.fz);
-    ud[0] = c * (a2 * q / g.r);
+    us[11] = c * (-a1 * (over(sd, g.R) - qy * cd) - a2 * q * g.fz);
+    ud[0] = c * (over(a2 * q, g.R));
     ud[1] = c * (g.tt / 2.0 + a2 * et * qx);
     ud[2] = c * (a1 * g.alx - a2 * q * qx);
-    ud[3] = c * (-a2 * xi * q / g.r3);
-    ud[4] = c * (-qy / 2.0 - a2 * et * q / g.r3);
-    ud[5] = c * (a1 / g.r + a2 * g.q2 / g.r3);
+    ud[3] = c * (over(-a2 * xi * q, g.R3));
+    ud[4] = c * (-qy / 2.0 - over(a2 * et * q, g.R3));
+    ud[5] = c * (over(a1, g.R) + over(a2 * g.q2, g.R3));
     ud[6] = c * (a2 * g.ey);
     ud[7] = c * (a1 * g.d * g.x11 + xy / 2.0 * sd + a2 * et * g.gy);
     ud[8] = c * (a1 * g.y * g.x11 - a2 * q * g.gy);
@@ -128,9 +168,10 @@ __device__ __forceinline__ void dc_ub2(const OkadaMedium &M, const OkadaSource &
     const double sd = S.sd, cd = S.cd, a3 = M.alp3, sdcd = S.sdcd, cdcd = S.cdcd;
     const double r = g.r, y = g.y, d = g.d;
     const double rd = r + d;
-    const double d11 = 1.0 / (r * rd);
-    const double aj2 = xi * y / rd * d11;
-    const double aj5 = -(d + y * y / rd) * d11;
+    const Divisor RD = divisor(rd), CD = {cd, S.icd};
+    const double d11 = over(1.0, {r * rd, g.R.inv * RD.inv});
+    const double aj2 = over(xi * y, RD) * d11;
+    const double aj5 = -(d + over(y * y, RD)) * d11;
     double ai3, ai4, ak1, ak3, aj3, aj6;
     if (cd != 0.0) {
         if (xi == 0.0) {
@@ -142,23 +183,24 @@ __device__ __forceinline__ void dc_ub2(const OkadaMedium &M, const OkadaSource &
                                              / (xi * (r + x) * cd)));
         }
         ai3 = (y * cd / rd - g.ale + sd * log(rd)) / cdcd;
-        ak1 = xi * (d11 - g.y11 * sd) / cd;
-        ak3 = (q * g.y11 - y * d11) / cd;
-        aj3 = (ak1 - aj2 * sd) / cd;
-        aj6 = (ak3 - aj5 * sd) / cd;
+        ak1 = over(xi * (d11 - g.y11 * sd), CD);
+        ak3 = over(q * g.y11 - y * d11, CD);
+        aj3 = over(ak1 - aj2 * sd, CD);
+        aj6 = over(ak3 - aj5 * sd, CD);
     } else {
-        double rd2 = rd * rd;
+        const double rd2 = rd * rd;
+        const Divisor RD2 = {rd2, RD.inv * RD.inv};
         ai3 = (et / rd + y * q / rd2 - g.ale) / 2.0;
         ai4 = xi * y / rd2 / 2.0;
-        ak1 = xi * q / rd * d11;
-        ak3 = sd / rd * (g.xi2 * d11 - 1.0);
-        aj3 = -xi / rd2 * (g.q2 * d11 - 1.0 / 2.0);
-        aj6 = -y / rd2 * (g.xi2 * d11 - 1.0 / 2.0);
+        ak1 = over(xi * q, RD) * d11;
+        ak3 = over(sd, RD) * (g.xi2 * d11 - 1.0);
+        aj3 = over(-xi, RD2) * (g.q2 * d11 - 1.0 / 2.0);
+        aj6 = over(-y, RD2) * (g.xi2 * d11 - 1.0 / 2.0);
     }
     const double xy = xi * g.y11;
     const double ai1 = -xi / rd * cd - ai4 * sd;
     const double ai2 = log(rd) + ai3 * sd;
-    const double ak2 = 1.0 / r + ak3 * sd;
+    const double ak2 = over(1.0, g.R) + ak3 * sd;
     const double ak4 = xy * cd - ak1 * sd;
     const double aj1 = aj5 * cd - aj6 * sd;
     const double aj4 = -xy - aj2 * cd + aj3 * sd;
@@ -167,10 +209,10 @@ __device__ __forceinline__ void dc_ub2(const OkadaMedium &M, const OkadaSource &
     us[1] = c * (-q / r + a3 * y / rd * sd);
     us[2] = c * (q * qy - a3 * ai2 * sd);
     us[3] = c * (g.xi2 * q * g.y32 - a3 * aj1 * sd);
-    us[4] = c * (xi * q / g.r3 - a3 * aj2 * sd);
+    us[4] = c * (over(xi * q, g.R3) - a3 * aj2 * sd);
     us[5] = c * (-xi * g.q2 * g.y32 - a3 * aj3 * sd);
     us[6] = c * (-xi * g.fy - d * g.x11 + a3 * (xy + aj4) * sd);
-    us[7] = c * (-g.ey + a3 * (1.0 / r + aj5) * sd);
+    us[7] = c * (-g.ey + a3 * (over(1.0, g.R) + aj5) * sd);
     us[8] = c * (q * g.fy - a3 * (qy - aj6) * sd);
     us[9] = c * (-xi * g.fz - y * g.x11 + a3 * ak1 * sd);
     us[10] = c * (-g.ez + a3 * y * d11 * sd);
@@ -178,9 +220,9 @@ __device__ __forceinline__ void dc_ub2(const OkadaMedium &M, const OkadaSource &
     ud[0] = c * (-q / r + a3 * ai3 * sdcd);
     ud[1] = c * (-et * qx - g.tt - a3 * xi / rd * sdcd);
     ud[2] = c * (q * qx + a3 * ai4 * sdcd);
-    ud[3] = c * (xi * q / g.r3 + a3 * aj4 * sdcd);
-    ud[4] = c * (et * q / g.r3 + qy + a3 * aj5 * sdcd);
-    ud[5] = c * (-g.q2 / g.r3 + a3 * aj6 * sdcd);
+    ud[3] = c * (over(xi * q, g.R3) + a3 * aj4 * sdcd);
+    ud[4] = c * (over(et * q, g.R3) + qy + a3 * aj5 * sdcd);
+    ud[5] = c * (over(-g.q2, g.R3) + a3 * aj6 * sdcd);
     ud[6] = c * (-g.ey + a3 * aj1 * sdcd);
     ud[7] = c * (-et * g.gy - xy * sd + a3 * aj2 * sdcd);
     ud[8] = c * (q * g.gy + a3 * aj3 * sdcd);
@@ -196,50 +238,50 @@ __device__ __forceinline__ void dc_uc2(const OkadaMedium &M, const OkadaSource &
 {
     const double cc = 1.0 / 6.283185307179586;
     const double sd = S.sd, cd = S.cd, a4 = M.alp4, a5 = M.alp5, sdsd = S.sdsd, sdcd = S.sdcd;
-    const double r = g.r, r2 = g.r2, r3 = g.r3, r5 = g.r5, y = g.y, d = g.d;
+    const double r = g.r, r2 = g.r2, y = g.y, d = g.d;
     const double xi2 = g.xi2, et2 = g.et2, q2 = g.q2, x11 = g.x11, y11 = g.y11;
     const double x32 = g.x32, y32 = g.y32;
     const double c = d + z;
-    const double x53 = (8.0 * r2 + 9.0 * r * xi + 3.0 * xi2) * x11 * x11 * x11 / r2;
-    const double y53 = (8.0 * r2 + 9.0 * r * et + 3.0 * et2) * y11 * y11 * y11 / r2;
+    const double x53 = over((8.0 * r2 + 9.0 * r * xi + 3.0 * xi2) * x11 * x11 * x11, g.R2);
+    const double y53 = over((8.0 * r2 + 9.0 * r * et + 3.0 * et2) * y11 * y11 * y11, g.R2);
     const double h = q * cd - z;
-    const double z32 = sd / r3 - h * y32;
-    const double z53 = 3.0 * sd / r5 - h * y53;
+    const double z32 = over(sd, g.R3) - h * y32;
+    const double z53 = over(3.0 * sd, g.R5) - h * y53;
     const double y0 = y11 - xi2 * y32;
     const double z0 = z32 - xi2 * z53;
-    const double ppy = cd / r3 + q * y32 * sd;
-    const double ppz = sd / r3 - q * y32 * cd;
+    const double ppy = over(cd, g.R3) + q * y32 * sd;
+    const double ppz = over(sd, g.R3) - q * y32 * cd;
     const double qq = z * y32 + z32 + z0;
-    const double qqy = 3.0 * c * d / r5 - qq * sd;
-    const double qqz = 3.0 * c * y / r5 - qq * cd + q * y32;
+    const double qqy = over(3.0 * c * d, g.R5) - qq * sd;
+    const double qqz = over(3.0 * c * y, g.R5) - qq * cd + q * y32;
     const double xy = xi * y11, qy = q * y11;
-    const double qr = 3.0 * q / r5;
-    const double cdr = (c + d) / r3;
-    const double yy0 = y / r3 - y0 * cd;
+    const double qr = over(3.0 * q, g.R5);
+    const double cdr = over(c + d, g.R3);
+    const double yy0 = over(y, g.R3) - y0 * cd;
     (void)y53;
     us[0] = cc * (a4 * xy * cd - a5 * xi * q * z32);
-    us[1] = cc * (a4 * (cd / r + 2.0 * qy * sd) - a5 * c * q / r3);
-    us[2] = cc * (a4 * qy * cd - a5 * (c * et / r3 - z * y11 + xi2 * z32));
+    us[1] = cc * (a4 * (over(cd, g.R) + 2.0 * qy * sd) - over(a5 * c * q, g.R3));
+    us[2] = cc * (a4 * qy * cd - a5 * (over(c * et, g.R3) - z * y11 + xi2 * z32));
     us[3] = cc * (a4 * y0 * cd - a5 * q * z0);
-    us[4] = cc * (-a4 * xi * (cd / r3 + 2.0 * q * y32 * sd) + a5 * c * xi * qr);
-    us[5] = cc * (-a4 * xi * q * y32 * cd + a5 * xi * (3.0 * c * et / r5 - qq));
+    us[4] = cc * (-a4 * xi * (over(cd, g.R3) + 2.0 * q * y32 * sd) + a5 * c * xi * qr);
+    us[5] = cc * (-a4 * xi * q * y32 * cd + a5 * xi * (over(3.0 * c * et, g.R5) - qq));
     us[6] = cc * (-a4 * xi * ppy * cd - a5 * xi * qqy);
-    us[7] = cc * (a4 * 2.0 * (d / r3 - y0 * sd) * sd - y / r3 * cd
-                  - a5 * (cdr * sd - et / r3 - c * y * qr));
-    us[8] = cc * (-a4 * q / r3 + yy0 * sd + a5 * (cdr * cd + c * d * qr - (y0 * cd + q * z0) * sd));
+    us[7] = cc * (a4 * 2.0 * (over(d, g.R3) - y0 * sd) * sd - over(y, g.R3) * cd
+                  - a5 * (cdr * sd - over(et, g.R3) - c * y * qr));
+    us[8] = cc * (over(-a4 * q, g.R3) + yy0 * sd + a5 * (cdr * cd + c * d * qr - (y0 * cd + q * z0) * sd));
     us[9] = cc * (a4 * xi * ppz * cd - a5 * xi * qqz);
-    us[10] = cc * (a4 * 2.0 * (y / r3 - y0 * cd) * sd + d / r3 * cd - a5 * (cdr * cd + c * d * qr));
+    us[10] = cc * (a4 * 2.0 * (over(y, g.R3) - y0 * cd) * sd + over(d, g.R3) * cd - a5 * (cdr * cd + c * d * qr));
     us[11] = cc * (yy0 * cd - a5 * (cdr * sd - c * y * qr - y0 * sdsd + q * z0 * cd));
-    ud[0] = cc * (a4 * cd / r - qy * sd - a5 * c * q / r3);
+    ud[0] = cc * (over(a4 * cd, g.R) - qy * sd - over(a5 * c * q, g.R3));
     ud[1] = cc * (a4 * y * x11 - a5 * c * et * q * x32);
     ud[2] = cc * (-d * x11 - xy * sd - a5 * c * (x11 - q2 * x32));
-    ud[3] = cc * (-a4 * xi / r3 * cd + a5 * c * xi * qr + xi * q * y32 * sd);
-    ud[4] = cc * (-a4 * y / r3 + a5 * c * et * qr);
-    ud[5] = cc * (d / r3 - y0 * sd + a5 * c / r3 * (1.0 - 3.0 * q2 / r2));
-    ud[6] = cc * (-a4 * et / r3 + y0 * sdsd - a5 * (cdr * sd - c * y * qr));
+    ud[3] = cc * (over(-a4 * xi, g.R3) * cd + a5 * c * xi * qr + xi * q * y32 * sd);
+    ud[4] = cc * (over(-a4 * y, g.R3) + a5 * c * et * qr);
+    ud[5] = cc * (over(d, g.R3) - y0 * sd + over(a5 * c, g.R3) * (1.0 - over(3.0 * q2, g.R2)));
+    ud[6] = cc * (over(-a4 * et, g.R3) + y0 * sdsd - a5 * (cdr * sd - c * y * qr));
     ud[7] = cc * (a4 * (x11 - y * y * x32) - a5 * c * ((d + 2.0 * q * cd) * x32 - y * et * q * x53));
     ud[8] = cc * (xi * ppy * sd + y * d * x32 + a5 * c * ((y + 2.0 * q * sd) * x32 - y * q2 * x53));
-    ud[9] = cc * (-q / r3 + y0 * sdcd - a5 * (cdr * cd + c * d * qr));
+    ud[9] = cc * (over(-q, g.R3) + y0 * sdcd - a5 * (cdr * cd + c * d * qr));
     ud[10] = cc * (a4 * y * d * x32 - a5 * c * ((y - 2.0 * q * sd) * x32 + d * et * q * x53));
     ud[11] = cc * (-xi * ppz * sd + x11 - d * d * x32
                    - a5 * c * ((d - 2.0 * q * cd) * x32 - d * q2 * x53));
