@@ -251,6 +251,8 @@ static void free_work(ucy_ctx *c)
     if (c->work) hipFree(c->work);
     c->work = nullptr;
     c->work_dim = 0;
+    if (c->h_step) hipHostFree(c->h_step);
+    c->h_step = nullptr;
 }
 
 extern "C" void ucy_destroy(ucy_ctx *c)
@@ -1326,6 +1328,18 @@ static int ensure_work(ucy_ctx *c)
     return 0;
 }
 
+// The pinned exchange buffer of ucy_odefun, ucy_rkck and ucy_rkqs: y and dydt (or
+// the candidate and its error) are neighbours on the device too, one copy each way.
+// From pageable arrays each of the 6 copies of a step of 945 patches waited for its
+// own staging: 250 us a step, with the launches of launch_rkck 200.  One call at a
+// time uses it, as all work buffers of a context.
+static int ensure_step(ucy_ctx *c, int n)
+{
+    if (c->h_step) return 0;
+    HIPCHK(hipHostMalloc((void **)&c->h_step, sizeof(double) * (2 * (size_t)n + 1)));
+    return 0;
+}
+
 static int check_ready(ucy_ctx *c, int n)
 {
     if (!c) return UCY_ERR_ARG;
@@ -1511,17 +1525,23 @@ extern "C" int ucy_odefun(ucy_ctx *c, int n, double time, const double *y, doubl
     (void)time;  // odefun does not depend on time (ratestate.f90:624-778)
     int rc = check_ready(c, n);
     if (rc) return rc;
+    if ((rc = ensure_step(c, n))) return rc;
     const PlainDims d = dims(c);
     RkBuffers &b = c->rb;
     double *d_vmax = b.t + d.m;  // spare slot after t
-    HIPCHK(hipMemcpyAsync(b.ytmp, y, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+    memcpy(c->h_step, y, sizeof(double) * n);
+    HIPCHK(hipMemcpyAsync(b.ytmp, c->h_step, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemsetAsync(d_vmax, 0, sizeof(double), c->stream));
     launch_prepass(c->stream, d, c->d_fr, c->d_rh, b.ytmp, b.ak[2], b.v, d_vmax);
     launch_gemv_post(c->stream, d, c->K, c->d_fr, b.ytmp, b.v, b.ak[2], b.t);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(dydt, b.ak[2], sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-    if (vmax) HIPCHK(hipMemcpyAsync(vmax, d_vmax, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    double *out = c->h_step + n, *out_vmax = out + n;
+    HIPCHK(hipMemcpyAsync(out, b.ak[2], sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+    if (vmax)
+        HIPCHK(hipMemcpyAsync(out_vmax, d_vmax, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    memcpy(dydt, out, sizeof(double) * n);
+    if (vmax) *vmax = *out_vmax;
     return UCY_OK;
 }
 
@@ -1561,16 +1581,22 @@ extern "C" int ucy_odefun_dev_static(ucy_ctx *c, int n, const double *y_dev, dou
     return UCY_OK;
 }
 
-// one Cash-Karp attempt on device buffers (y, dydt already resident)
-static void rkck_device(ucy_ctx *c, const PlainDims &d, double h)
+// y and dydt to the device; the candidate and its error back, behind all that the
+// stream holds
+static int step_in(ucy_ctx *c, int n, const double *y, const double *dydt)
 {
-    RkBuffers &b = c->rb;
-    for (int s = 2; s <= 6; s++) {
-        launch_rk_combine(c->stream, d.dim, s, h, b.y, b.ak, nullptr, b.ytmp, nullptr, nullptr);
-        launch_prepass(c->stream, d, c->d_fr, c->d_rh, b.ytmp, b.ak[s], b.v, nullptr);
-        launch_gemv_post(c->stream, d, c->K, c->d_fr, b.ytmp, b.v, b.ak[s], nullptr);
-    }
-    launch_rk_combine(c->stream, d.dim, 7, h, b.y, b.ak, nullptr, nullptr, b.ycand, b.yerr);
+    memcpy(c->h_step, y, sizeof(double) * n);
+    memcpy(c->h_step + n, dydt, sizeof(double) * n);
+    HIPCHK(hipMemcpyAsync(c->rb.y, c->h_step, sizeof(double) * 2 * n, hipMemcpyHostToDevice,
+                          c->stream));
+    return 0;
+}
+static int step_out(ucy_ctx *c, int n)
+{
+    HIPCHK(hipMemcpyAsync(c->h_step, c->rb.ycand, sizeof(double) * 2 * n, hipMemcpyDeviceToHost,
+                          c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return 0;
 }
 
 extern "C" int ucy_rkck(ucy_ctx *c, int n, double t, const double *yin, const double *dydt,
@@ -1579,15 +1605,15 @@ extern "C" int ucy_rkck(ucy_ctx *c, int n, double t, const double *yin, const do
     (void)t;
     int rc = check_ready(c, n);
     if (rc) return rc;
+    if ((rc = ensure_step(c, n))) return rc;
     const PlainDims d = dims(c);
     RkBuffers &b = c->rb;
-    HIPCHK(hipMemcpyAsync(b.y, yin, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(b.dydt, dydt, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-    rkck_device(c, d, h);
+    if ((rc = step_in(c, n, yin, dydt))) return rc;
+    launch_rkck(c->stream, d, c->K, c->d_fr, c->d_rh, b, h);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(yout, b.ycand, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(yerr, b.yerr, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if ((rc = step_out(c, n))) return rc;
+    memcpy(yout, c->h_step, sizeof(double) * n);
+    memcpy(yerr, c->h_step + n, sizeof(double) * n);
     return UCY_OK;
 }
 
@@ -1599,19 +1625,18 @@ extern "C" int ucy_rkqs(ucy_ctx *c, int n, double *t, double *y, double *dydt,
 {
     int rc = check_ready(c, n);
     if (rc) return rc;
+    if ((rc = ensure_step(c, n))) return rc;
     const PlainDims d = dims(c);
     RkBuffers &b = c->rb;
-    HIPCHK(hipMemcpyAsync(b.y, y, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(b.dydt, dydt, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-    std::vector<double> yerr(n), ycand(n);
+    if ((rc = step_in(c, n, y, dydt))) return rc;
+    // the candidate comes with the error, which most attempts accept
+    const double *ycand = c->h_step, *yerr = c->h_step + n;
     const double SAFETY = 0.7, PGROW = -0.2, PSHRNK = -0.15, ERRCON = 1.89e-4;
     double h = htry;
     for (;;) {
-        rkck_device(c, d, h);
+        launch_rkck(c->stream, d, c->K, c->d_fr, c->d_rh, b, h);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(yerr.data(), b.yerr, sizeof(double) * n, hipMemcpyDeviceToHost,
-                              c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
+        if ((rc = step_out(c, n))) return rc;
         double errmax = 0.0;
         for (int i = 0; i < n; i++) {
             const double e = fabs(yerr[i] / yscal[i]);
@@ -1626,8 +1651,7 @@ extern "C" int ucy_rkqs(ucy_ctx *c, int n, double *t, double *y, double *dydt,
             if (*hnext > max_step) *hnext = max_step;
             *hdid = h;
             *t = *t + h;
-            HIPCHK(hipMemcpyAsync(y, b.ycand, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(hipStreamSynchronize(c->stream));
+            memcpy(y, ycand, sizeof(double) * n);
             return UCY_OK;
         }
     }

@@ -322,6 +322,23 @@ void launch_start(hipStream_t st, const PlainDims &d, const Friction *fr, const 
     hipLaunchKernelGGL(start_kernel, dim3((ne + 255) / 256), dim3(256), 0, st, d, fr, rh, b, ctl);
 }
 
+// the N state entries from so on of the input of stage `stage`.  All loads before
+// the stores, which may alias them: entry by entry each waited for the last one's
+// memory (a stage of 945 patches 12.9 us at best, so 11.3).
+template <int N>
+__device__ __forceinline__ void stage_entries(const RkBuffers &b, double h, int so, int stage)
+{
+    double v[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const int i = so + k;
+        v[k] = stage_value(stage, h, b.y[i], b.dydt[i], b.ak[2][i], b.ak[3][i], b.ak[4][i],
+                           b.ak[5][i]);
+    }
+#pragma unroll
+    for (int k = 0; k < N; k++) b.ytmp[so + k] = v[k];
+}
+
 // the input of stage `stage` (2..6) for element e and its pre-pass; the
 // slip-rate entries go to vout (less v0 in the reduced paths)
 __device__ __forceinline__ void stage_elem(const PlainDims &d, const Friction *__restrict__ fr,
@@ -329,11 +346,12 @@ __device__ __forceinline__ void stage_elem(const PlainDims &d, const Friction *_
                                            double h, int e, int stage, double *vout)
 {
     const int so = elem_state_off(d, e), vo = elem_v_off(d, e);
-    const int ns = elem_nstate(d, e);
-    for (int k = 0; k < ns; k++) {
-        const int i = so + k;
-        b.ytmp[i] = stage_value(stage, h, b.y[i], b.dydt[i], b.ak[2][i], b.ak[3][i], b.ak[4][i],
-                                b.ak[5][i]);
+    switch (elem_nstate(d, e)) {
+    case 4: stage_entries<4>(b, h, so, stage); break;
+    case 5: stage_entries<5>(b, h, so, stage); break;
+    case 6: stage_entries<6>(b, h, so, stage); break;
+    case 7: stage_entries<7>(b, h, so, stage); break;
+    default: stage_entries<12>(b, h, so, stage); break;
     }
     double *out = b.ak[stage];
     if (d.ps && e >= d.np) ps_volume_prepass(b.ytmp + so, rh[e - d.np], out + so, vout + vo);
@@ -577,41 +595,88 @@ void launch_commit(hipStream_t st, int dim, const RkBuffers &b, Control *ctl)
 }
 
 // ---------------------------------------------------------------------------
-// standalone stage combination for ucy_rkck: stage 2..6 writes ytmp, stage 7
-// writes yout and yerr.
+// One Cash-Karp evaluation for a host's own step loop (ucy_rkck, ucy_rkqs): the
+// caller's h and k1, binary64 K whatever the context integrates with.  A launch
+// per stage: as in the captured attempt a matvec's wave makes its element's next
+// stage input, so that a step has 6 launches where combination, pre-pass and matvec
+// apart made 16.  Bound by K from the last-level cache: 945 patches (43 MB) take
+// TODO us per stage.
 // ---------------------------------------------------------------------------
-__global__ void rk_combine_kernel(int n, int stage, double h, const double *__restrict__ yin,
-                                  const double *k1, const double *k2, const double *k3,
-                                  const double *k4, const double *k5, const double *k6,
-                                  double *ytmp, double *yout, double *yerr)
+__global__ void __launch_bounds__(64)
+rkck_begin_kernel(PlainDims d, const Friction *__restrict__ fr, const Rheology *__restrict__ rh,
+                  RkBuffers b, double h)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (stage <= 6) {
-        ytmp[i] = stage_value(stage, h, yin[i], k1[i], stage > 2 ? k2[i] : 0.0,
-                              stage > 3 ? k3[i] : 0.0, stage > 4 ? k4[i] : 0.0,
-                              stage > 5 ? k5[i] : 0.0);
-        return;
-    }
-    double yr = C1 * k1[i];
-    yr = yr + C3 * k3[i];
-    yr = yr + C4 * k4[i];
-    yr = yr + C6 * k6[i];
-    yout[i] = yin[i] + h * yr;
-    double e = DC1 * k1[i];
-    e = e + DC3 * k3[i];
-    e = e + DC4 * k4[i];
-    e = e + DC5 * k5[i];
-    e = e + DC6 * k6[i];
-    yerr[i] = h * e;
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < d.np + d.nv) stage_elem(d, fr, rh, b, h, e, 2, b.v2);
 }
 
-void launch_rk_combine(hipStream_t st, int n, int stage, double h, const double *yin,
-                       double *const *ak, double *yr, double *ytmp, double *yout, double *yerr)
+// N entries of the fifth-order solution and of the error (ode45.f90:190-200)
+template <int N>
+__device__ __forceinline__ void step_entries(const RkBuffers &b, double h, int so)
 {
-    (void)yr;
-    hipLaunchKernelGGL(rk_combine_kernel, dim3((n + 255) / 256), dim3(256), 0, st, n, stage, h,
-                       yin, ak[1], ak[2], ak[3], ak[4], ak[5], ak[6], ytmp, yout, yerr);
+    double y[N], err[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const int i = so + k;
+        const double k1 = b.dydt[i], k3 = b.ak[3][i], k4 = b.ak[4][i], k5 = b.ak[5][i],
+                     k6 = b.ak[6][i];
+        double yr = C1 * k1;
+        yr = yr + C3 * k3;
+        yr = yr + C4 * k4;
+        yr = yr + C6 * k6;
+        y[k] = b.y[i] + h * yr;
+        double er = DC1 * k1;
+        er = er + DC3 * k3;
+        er = er + DC4 * k4;
+        er = er + DC5 * k5;
+        er = er + DC6 * k6;
+        err[k] = h * er;
+    }
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        b.ycand[so + k] = y[k];
+        b.yerr[so + k] = err[k];
+    }
+}
+
+// stage 2..5: k_stage, then the input of the next stage; 6: k_6, then the
+// fifth-order solution and the error
+__global__ void __launch_bounds__(256)
+rkck_stage_kernel(PlainDims d, KOperand K, const Friction *__restrict__ fr,
+                  const Rheology *__restrict__ rh, RkBuffers b, double h, int stage)
+{
+    const int lane = threadIdx.x & 63;
+    const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (e >= d.np + d.nv) return;
+    const double *vin = (stage & 1) ? b.v : b.v2;
+    double *vout = (stage & 1) ? b.v2 : b.v;
+    elem_gemv_post<DOT_F64>(d, K, fr, b.ytmp, vin, b.ak[stage], nullptr, e, lane, nullptr, nullptr,
+                            nullptr);
+    if (lane != 0) return;
+    if (stage < 6) {
+        stage_elem(d, fr, rh, b, h, e, stage + 1, vout);
+        return;
+    }
+    const int so = elem_state_off(d, e);
+    switch (elem_nstate(d, e)) {
+    case 4: step_entries<4>(b, h, so); break;
+    case 5: step_entries<5>(b, h, so); break;
+    case 6: step_entries<6>(b, h, so); break;
+    case 7: step_entries<7>(b, h, so); break;
+    default: step_entries<12>(b, h, so); break;
+    }
+}
+
+void launch_rkck(hipStream_t st, const PlainDims &d, const double *K, const Friction *fr,
+                 const Rheology *rh, RkBuffers b, double h)
+{
+    const int ne = d.np + d.nv;
+    b.v0 = nullptr;   // slip rates themselves, not their increments
+    const KOperand k{K, nullptr, nullptr, 0};
+    hipLaunchKernelGGL(rkck_begin_kernel, dim3((ne + 63) / 64), dim3(64), 0, st, d, fr, rh, b, h);
+    for (int s = 2; s <= 6; s++)
+        hipLaunchKernelGGL(rkck_stage_kernel, dim3((ne + 3) / 4), dim3(256), 0, st, d, k, fr, rh, b,
+                           h, s);
 }
 
 }  // namespace ucy

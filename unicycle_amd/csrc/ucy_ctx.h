@@ -73,6 +73,7 @@ struct ucy_ctx {
     // work buffers
     double *work = nullptr;
     size_t work_dim = 0;
+    double *h_step = nullptr;  // pinned: the states that a host's own step loop exchanges
     RkBuffers rb{};
     Control *d_ctl = nullptr;
     Control *h_ctl = nullptr;  // pinned

@@ -179,7 +179,7 @@ void launch_obs_log(hipStream_t st, const RkBuffers &b, Control *ctl);
 void launch_disp_gemv(hipStream_t st, const double *O, int64_t rows, int64_t n, int np, int model,
                       const double *y, double *d, double *df, double *dl, const Control *ctl);
 // standalone Cash-Karp combination kernels for the ucy_rkck entry point
-void launch_rk_combine(hipStream_t st, int n, int stage, double h, const double *yin,
-                       double *const *ak, double *yr, double *ytmp, double *yout, double *yerr);
+void launch_rkck(hipStream_t st, const PlainDims &d, const double *K, const Friction *fr,
+                 const Rheology *rh, RkBuffers b, double h);
 
 }  // namespace ucy
