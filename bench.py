@@ -74,13 +74,10 @@ INF_T = 1e30               # no end time: runs are bounded by attempts
 MEASURED_TRAFFIC = {"split_bf16": 2.269e9, "bf16_i8": 1.733e9}
 # FP64 flop per (receiver, source) pair of the assembly kernels from
 # rocprofv3 --pmc SQ_INSTS_VALU_FLOPS_FP64 x 64 lanes / pairs on the same
-# models (profiles/assembly_greens_functions.md).  The strain-volume figure
-# is the evaluation that forms every displacement-gradient entry once; the
-# device kernel splits it by displacement component and executes
-# EXECUTED_FLOP_PER_PAIR (ADD + MUL + 2 FMA + TRANS counters), reported beside it
-ASSEMBLY_FLOP_PER_PAIR = {"okada": 7108.0, "okada_stress": 7199.0, "nikkhoo": 21680.0,
-                          "strain_volume": 61800.0}
-EXECUTED_FLOP_PER_PAIR = {"strain_volume": 106700.0}
+# models (profiles/assembly_greens_functions.md); strain volumes: patch and volume
+# receivers in the model's proportion
+ASSEMBLY_FLOP_PER_PAIR = {"okada": 5161.0, "okada_stress": 5251.0, "nikkhoo": 12875.0,
+                          "strain_volume": 10315.0}
 FP64_VALU_PEAK = 78.6e12   # FLOP/s, dense binary64 vector
 
 
@@ -739,10 +736,6 @@ def bench_assembly(args, cpu=True):
         r = {"bound": "fp64 valu", "achieved": a / 1e12, "peak": FP64_VALU_PEAK / 1e12,
              "unit": "TFLOP/s", "frac": a / FP64_VALU_PEAK,
              "flop_per_pair": ASSEMBLY_FLOP_PER_PAIR[key]}
-        if key in EXECUTED_FLOP_PER_PAIR:
-            x = pairs_per_s * EXECUTED_FLOP_PER_PAIR[key]
-            r.update({"executed_flop_per_pair": EXECUTED_FLOP_PER_PAIR[key],
-                      "executed_achieved": x / 1e12, "executed_frac": x / FP64_VALU_PEAK})
         return r
 
     out["okada_rectangles"] = {"elements": N, "pairs": N * N, "K_bytes": kb, "gpu_s": secs[0],

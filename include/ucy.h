@@ -328,9 +328,10 @@ int ucy_rkck(ucy_ctx *ctx, int n, double t, const double *yin, const double *dyd
 int ucy_rkqs(ucy_ctx *ctx, int n, double *t, double *y, double *dydt, const double *yscal,
              double htry, double *hdid, double *hnext, double epsilon, double max_step);
 
-/* Main loop of ratestate.f90:307-328 run device-resident: one graph-captured
- * RK45 attempt per replay, state kept in HBM.  y is read at entry and written
- * at exit.  Optional logs receive, per accepted step, the time reached, dt_done
+/* Main loop of ratestate.f90:307-328 run device-resident: many RK45 attempts
+ * per launch of a resident kernel, or (K beyond 1 GB in binary64, 2 GB reduced,
+ * or no room on the device for the resident blocks) one graph-captured attempt
+ * per replay, with the same bits.  y is read at entry and written at exit.  Optional logs receive, per accepted step, the time reached, dt_done
  * and the vMax of the step-start odefun (ratestate.f90:530-532). */
 typedef struct {
     double time;        /* simulated time reached */
@@ -465,8 +466,9 @@ int ucy_ensemble_matvec(ucy_ensemble *ens, int group, const double *V, double *T
  * and decoded once per block into LDS), and its table of seconds
  * per launch (UCY_GEMM_TUNE_ENTRIES entries: k-blocks 32, 48, 64, 80, 96,
  * 104, 128, 160, 192, 256, 512 of variant 0, then of 1, ...; -1 = not
- * admissible); pointers may be NULL.  The tuner takes the candidate with the
- * least launch time plus the post-passes' read of its split partial
+ * admissible); pointers may be NULL.  Ensembles whose launch has fewer than 256
+ * blocks at 32 k-blocks are also timed at 2 to 24, outside the table.  The tuner
+ * takes the candidate with the least launch time plus the post-passes' read of its split partial
  * products charged at 4 TB/s. */
 #define UCY_GEMM_TUNE_ENTRIES 121
 /* override the autotuner: k-blocks per split and split-bf16 variant (as in

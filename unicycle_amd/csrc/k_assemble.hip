@@ -44,8 +44,8 @@ __device__ __forceinline__ void proj_volume(const Receiver &R, const double S[6]
     o[5] = -c1 * dv[0] - c2 * dv[1] - c3 * dv[2];
 }
 
-// Bound by binary64 arithmetic and its latencies: some 11 thousand instructions
-// per wave of pairs.  Two waves per SIMD (28 registers to scratch) hide more than
+// Bound by binary64 arithmetic and its latencies: 5.0 thousand instructions per
+// wave of pairs, 71 % of the issue slots.  Two waves per SIMD (28 registers to scratch) hide more than
 // they cost: 2048 sources on themselves take 0.85 ms, at one wave (276 registers)
 // 0.94, and with divisions in place of the corrected reciprocals of okada_dev.h
 // 1.09 and 1.30.

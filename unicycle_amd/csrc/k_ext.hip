@@ -216,11 +216,11 @@ __device__ __forceinline__ void sv_store(const Receiver &R, const double st[6][6
             for (int c = 0; c < NC; c++) out[(int64_t)(e * NC + c) * out_stride + s] = o[e][c];
 }
 
-// Every pair off the faces' planes.  Bound by the issue of vector instructions,
-// some 15 thousand per wave of pairs (four laps of two corners), at 1 wave per
-// SIMD; the columns of K are 8 % of the time at 7 TB/s.  594 volumes on 234
-// patches and on themselves: 78 + 162 us; the formula text differentiated in
-// forward mode for every pair took 1.19 + 2.67 ms.
+// Every pair off the faces' planes.  Bound by the issue of vector instructions, 9.5
+// thousand per wave of pairs, at 1 wave per SIMD (74 % of the issue slots); the
+// columns of K are 8 % of the time at 7 TB/s.  594 volumes on 234 patches and on
+// themselves: 78 + 160 us; the formula text differentiated in forward mode for every
+// pair took 1.19 + 2.67 ms.  8192 volumes on themselves 21.7 ms, before 443.
 template <int KIND>
 __global__ void __launch_bounds__(64)
 sv_sums_kernel(SvMedium M, double G, double nu, double lambda, const SvSource *__restrict__ src,
