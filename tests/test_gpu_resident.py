@@ -95,6 +95,10 @@ MODELS = {
     "planestrain-volumes": lambda mk: _planestrain(mk, 24, 4, 3),
     "volumes": lambda mk: _volumes(mk, 7, 5, (3, 3, 2)),
     "volumes-large": lambda mk: _volumes(mk, 13, 7, (5, 5, 4)),
+    # more blocks than a volume's rows allow at equal cuts: ranges without an
+    # element are dropped from the plan
+    "volumes-39-200": lambda mk: _volumes(mk, 13, 3, (10, 5, 4)),
+    "volumes-390-50": lambda mk: _volumes(mk, 26, 15, (5, 5, 2)),
 }
 
 
@@ -131,7 +135,8 @@ def test_same_bits_as_the_captured_attempt(engine_factory, name):
     eng.close()
 
 
-@pytest.mark.parametrize("name", ["thrust-45", "thrust-247", "volumes"])
+@pytest.mark.parametrize("name", ["thrust-45", "thrust-247", "volumes", "volumes-large",
+                                  "volumes-39-200", "volumes-390-50"])
 @pytest.mark.parametrize("precision", [PREC_MIXED, PREC_SPLIT_BF16])
 def test_reduced_precision(engine_factory, name, precision):
     eng = MODELS[name](engine_factory)

@@ -1683,52 +1683,17 @@ static int capture_attempt(ucy_ctx *c)
     return 0;
 }
 
-// The resident integrator's blocks, their shares and LDS (k_resident.hip), with
-// its buffers in place.  0: planned; 1: the model takes the captured attempt;
-// < 0: an error.
-//   - Share of a block: 48 KB of K, so that a stage's products (0.2 us) take
-//     less than the exchange among the blocks (1.5 us with 8, 3.8 us with 256).
-//     8 to 72 KB measure within 10 % of each other; a reduced K has fewer bytes
-//     per row and takes 16 KB (200 patches: 28 us per attempt, 35 us at 48 KB).
-//   - One block where K fits it whole, as it needs no exchange.
-//   - At most 1 GB of K in binary64 (4096 patches: 755 us per attempt, captured
-//     770 us; 8192 patches: 2985 and 2910 us, the launches no longer show) and
-//     2 GB reduced (8192 patches: 1775 and 1800 us).
-//   - Rows beyond LDS up to 64 KB per CU are left to the L2 (1600 patches 103 us,
-//     109 us if all stream; 2816 patches 368 and 353 us).
+// The resident integrator's plan (resident_plan.h) with its buffers in place.
+// 0: planned; 1: the model takes the captured attempt; < 0: an error.
 static int plan_resident(ucy_ctx *c, const PlainDims &d, ResArgs &a, size_t &lds)
 {
-    constexpr int64_t kLds = 158 * 1024, kOneBlock = 96 * 1024, kCachedBytes = 64 * 1024;
     const bool f64 = c->kprec == UCY_PREC_F64;
-    const int64_t m = d.m, n = d.n, entry = f64 ? 8 : 4, kShare = (f64 ? 48 : 16) * 1024;
-    const int64_t kb = m * n * entry;
-    const int ne = d.np + d.nv;
-    if (kb > (f64 ? 1ll << 30 : 2ll << 30)) return 1;
-    int64_t P = kb <= kOneBlock && ne <= 64 ? 1 : std::max<int64_t>(2, (kb + kShare - 1) / kShare);
-    P = std::max<int64_t>(P, (ne + 55) / 56);
-    P = std::min<int64_t>(P, kResMaxBlocks);
-    // element boundaries at equal numbers of rows
-    const int64_t rp = d.ps ? 2 : d.ap ? 1 : 3, rv = d.ps ? 3 : d.ap ? 2 : 6;
-    std::vector<int> bounds(P + 1);
-    int el = 0, rows = 0;
-    for (int64_t b = 0; b <= P; b++) {
-        const int64_t r = m * b / P;
-        bounds[b] = (int)(r <= rp * d.np ? (r + rp - 1) / rp
-                                         : d.np + (r - rp * d.np + rv - 1) / rv);
-        if (b == 0) continue;
-        auto row = [&](int e) { return e <= d.np ? rp * e : rp * d.np + rv * (e - d.np); };
-        el = std::max(el, bounds[b] - bounds[b - 1]);
-        rows = std::max(rows, (int)(row(bounds[b]) - row(bounds[b - 1])));
-    }
-    if (el > 64) return 1;
-    el += el & 1;
-    rows += rows & 1;
-    const int64_t other = 8 * (n + 2ll * resident_state_entries(d) * el + 2ll * rows);
-    if (other > kLds) return 1;
-    const int64_t lr = std::min<int64_t>(rows, (kLds - other) / (n * entry));
-    lds = (size_t)(other + lr * n * entry);
+    const ResidentPlan plan = resident_plan(c->model, d.np, d.nv, d.m, d.n, f64);
+    if (!plan.P) return 1;
+    const int64_t P = plan.P;
+    lds = plan.lds;
     const size_t hb = 64, bb = 8 * (kResMaxBlocks / 2 + 1);
-    a.xbytes = 8 * 4 * (3 * (size_t)P + (size_t)n);
+    a.xbytes = 8 * 4 * (3 * (size_t)P + (size_t)d.n);
     int rc = ensure_buf(c, c->res, hb + bb + a.xbytes);
     if (rc) return rc;
     char *p = (char *)c->res.p;
@@ -1742,18 +1707,18 @@ static int plan_resident(ucy_ctx *c, const PlainDims &d, ResArgs &a, size_t &lds
     a.bounds = (const int *)(p + hb);
     a.red = (unsigned long long *)(p + hb + bb);
     a.v = a.red + 4 * 3 * P;
-    a.P = (int)P;
-    a.threads = P == 1 && m <= 8 ? 128 : kResThreads;
-    a.el_max = el;
-    a.rows_max = rows;
-    a.rows_lds = (int)lr;
-    a.rows_cached = (int)(lr + kCachedBytes / (n * entry));
+    a.P = plan.P;
+    a.threads = P == 1 && d.m <= 8 ? 128 : kResThreads;
+    a.el_max = plan.el_max;
+    a.rows_max = plan.rows_max;
+    a.rows_lds = plan.rows_lds;
+    a.rows_cached = plan.rows_cached;
     // launches of some 30 ms: 20 us and K's reading time per attempt
-    const double us = 20.0 + (double)kb / 1.0e6;
+    const double us = 20.0 + (double)d.m * d.n * (f64 ? 8 : 4) / 1.0e6;
     a.max_attempts = (int)std::max(16.0, std::min(2000.0, 30000.0 / us));
-    HIPCHK(hipMemcpyAsync((void *)a.bounds, bounds.data(), sizeof(int) * (P + 1),
+    HIPCHK(hipMemcpyAsync((void *)a.bounds, plan.bounds.data(), sizeof(int) * (P + 1),
                           hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));   // bounds is on this call's stack
+    HIPCHK(hipStreamSynchronize(c->stream));   // the plan is on this call's stack
     return 0;
 }
 

@@ -32,7 +32,10 @@
 // exchange is one way out and one way in.  Buffers go round in fours: when a
 // block publishes exchange k it has every block's k-1, so all have read k-2,
 // whose buffer it empties for k+2; the emptying is complete (s_waitcnt) before
-// it publishes k+1, and nobody polls k+2 without having that.  No plain load or
+// it publishes k+1, and nobody polls k+2 without having that.  This needs every
+// block to publish slip rates, so the plan has no block without an element
+// (resident_plan.h): nobody would wait for one within an attempt, and its buffer
+// would be emptied before it has read it.  No plain load or
 // store touches exchanged data, so no cache has to be written back or
 // invalidated: with agent-scope release and acquire fences an exchange took
 // 59-64 us; with these accesses and a flag per block 1.8 us among 32 blocks
@@ -650,11 +653,6 @@ static ResKernel resident_of(const PlainDims &d, int prec)
     if (d.ap) return resident_of<RES_ANTIPLANE>(prec);
     if (d.ps) return resident_of<RES_PLANESTRAIN>(prec);
     return d.nv ? resident_of<RES_VOLUME>(prec) : resident_of<RES_PATCH>(prec);
-}
-
-int resident_state_entries(const PlainDims &d)
-{
-    return d.ap ? 4 : d.ps ? 6 : d.nv ? 12 : 7;
 }
 
 hipError_t launch_resident(hipStream_t st, const ResArgs &a, size_t lds)

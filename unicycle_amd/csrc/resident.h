@@ -1,11 +1,11 @@
 // resident.h -- the resident integrator (k_resident.hip): its arguments and plan
 #pragma once
+#include "resident_plan.h"
 #include "ucy_internal.h"
 
 namespace ucy {
 
 constexpr int kResThreads = 512;      // at most, per block
-constexpr int kResMaxBlocks = 256;    // one per CU
 
 struct ResHead {
     unsigned arrived, state;          // state 0: forming, 1: complete, 2: given up
@@ -32,8 +32,6 @@ struct ResArgs {
     int max_attempts;
 };
 
-// state entries per element that the kernel holds in LDS, for its size
-int resident_state_entries(const PlainDims &d);
 hipError_t launch_resident(hipStream_t st, const ResArgs &a, size_t lds);
 
 }  // namespace ucy
