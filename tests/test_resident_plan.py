@@ -17,9 +17,9 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
                     "csrc")
 SOURCE = """
 #include "resident_plan.h"
-extern "C" int plan(int model, int np, int nv, long m, long n, int f64, int *bounds, long *size)
+extern "C" int plan(int model, int np, int nv, long m, long n, int f64, int cus, int *bounds, long *size)
 {
-    const ucy::ResidentPlan p = ucy::resident_plan(model, np, nv, m, n, f64);
+    const ucy::ResidentPlan p = ucy::resident_plan(model, np, nv, m, n, f64, cus);
     if (!p.P) return 0;
     for (size_t i = 0; i < p.bounds.size(); i++) bounds[i] = p.bounds[i];
     const long s[] = {(long)p.bounds.size(), p.el_max, p.rows_max, p.rows_lds, p.rows_cached,
@@ -45,26 +45,26 @@ def plan(tmp_path_factory):
     subprocess.run([cxx, "-std=c++17", "-O1", "-shared", "-fPIC", "-I", CSRC, str(d / "plan.cpp"),
                     "-o", str(d / "plan.so")], check=True)
     f = ctypes.CDLL(str(d / "plan.so")).plan
-    f.argtypes = [ctypes.c_int] * 3 + [ctypes.c_long] * 2 + [ctypes.c_int,
+    f.argtypes = [ctypes.c_int] * 3 + [ctypes.c_long] * 2 + [ctypes.c_int, ctypes.c_int,
                                                               ctypes.POINTER(ctypes.c_int),
                                                               ctypes.POINTER(ctypes.c_long)]
 
-    def call(model, np_, nv, f64):
+    def call(model, np_, nv, f64, cus=256):
         m = ROWS[model][0] * np_ + ROWS[model][1] * nv
         n = COLS[model][0] * np_ + COLS[model][1] * nv
         n += n & 1
         bounds, size = (ctypes.c_int * 300)(), (ctypes.c_long * 6)()
-        P = f(model, np_, nv, m, n, f64, bounds, size)
+        P = f(model, np_, nv, m, n, f64, cus, bounds, size)
         return m, n, P, list(bounds[:P + 1]), list(size)
     return call
 
 
-def _check(plan, model, np_, nv, f64):
-    m, n, P, b, (count, el, rows, lds_rows, cached, lds) = plan(model, np_, nv, f64)
+def _check(plan, model, np_, nv, f64, cus=256):
+    m, n, P, b, (count, el, rows, lds_rows, cached, lds) = plan(model, np_, nv, f64, cus)
     if not P:
         return False
-    what = (model, np_, nv, f64)
-    assert P <= 256 and count == P + 1 and b[0] == 0 and b[-1] == np_ + nv, what
+    what = (model, np_, nv, f64, cus)
+    assert P <= min(cus, 256) and count == P + 1 and b[0] == 0 and b[-1] == np_ + nv, what
     assert all(x < y for x, y in zip(b, b[1:])), (what, "a block without an element")
     rp, rv = ROWS[model]
     first = [rp * min(e, np_) + rv * max(e - np_, 0) for e in b]
@@ -86,6 +86,16 @@ def test_every_block_has_an_element(plan, model, f64):
     sizes += [(int(a), int(b)) for a, b in np.exp(rng.uniform(0.0, np.log(2500.0), (1500, 2)))]
     planned = sum(_check(plan, model, np_, nv, f64) for np_, nv in sizes)
     assert planned > len(sizes) // 2
+
+
+@pytest.mark.parametrize("cus", [1, 32, 64, 304])
+def test_at_most_a_block_per_cu(plan, cus):
+    """A device partition has fewer CUs; more elements than its blocks take are
+    left to the captured attempt."""
+    for f64 in (True, False):
+        planned = [_check(plan, 0, np_, nv, f64, cus)
+                   for np_, nv in [(20, 0), (390, 0), (945, 0), (39, 200), (2048, 0), (4096, 0)]]
+        assert planned == [n <= 64 * cus for n in (20, 390, 945, 239, 2048, 4096)]
 
 
 def test_limits(plan):

@@ -223,7 +223,8 @@ extern "C" ucy_ctx *ucy_create(int device, int flags)
     (void)flags;
     ucy_ctx *c = new ucy_ctx();
     c->device = device;
-    if (hipSetDevice(device) != hipSuccess) {
+    if (hipSetDevice(device) != hipSuccess ||
+        hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
         delete c;
         return nullptr;
     }
@@ -1688,7 +1689,7 @@ static int capture_attempt(ucy_ctx *c)
 static int plan_resident(ucy_ctx *c, const PlainDims &d, ResArgs &a, size_t &lds)
 {
     const bool f64 = c->kprec == UCY_PREC_F64;
-    const ResidentPlan plan = resident_plan(c->model, d.np, d.nv, d.m, d.n, f64);
+    const ResidentPlan plan = resident_plan(c->model, d.np, d.nv, d.m, d.n, f64, c->cus);
     if (!plan.P) return 1;
     const int64_t P = plan.P;
     lds = plan.lds;

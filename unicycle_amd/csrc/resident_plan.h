@@ -8,7 +8,7 @@
 
 namespace ucy {
 
-constexpr int kResMaxBlocks = 256;    // one per CU
+constexpr int kResMaxBlocks = 256;    // one per CU of a whole MI355X
 constexpr int kResMaxElements = 64;   // of a block: one lane of wave 0 each
 
 enum { RES_MODEL_3D = 0, RES_MODEL_ANTIPLANE = 1, RES_MODEL_PLANESTRAIN = 2 };
@@ -29,7 +29,10 @@ struct ResidentPlan {
 };
 
 // np patches, nv volumes, K of m rows and n columns (as stored, n even) with
-// binary64 entries (f64) or packed words of 4 bytes.
+// binary64 entries (f64) or packed words of 4 bytes, on a device of cus CUs.
+//   - At most a block per CU, as all are resident at once and a block's LDS is most
+//     of a CU's.  A device partition has fewer CUs than the whole: blocks beyond
+//     them would find no room, and each call would wait 2 ms to learn it.
 //   - Share of a block: 48 KB of K, so that a stage's products (0.2 us) take
 //     less than the exchange among the blocks (1.5 us with 8, 3.8 us with 256).
 //     8 to 72 KB measure within 10 % of each other; a reduced K has fewer bytes
@@ -44,7 +47,8 @@ struct ResidentPlan {
 //     2 GB reduced (8192 patches: 1775 and 1800 us).
 //   - Rows beyond LDS up to 64 KB per CU are left to the L2 (1600 patches 103 us,
 //     109 us if all stream; 2816 patches 368 and 353 us).
-inline ResidentPlan resident_plan(int model, int np, int nv, int64_t m, int64_t n, bool f64)
+inline ResidentPlan resident_plan(int model, int np, int nv, int64_t m, int64_t n, bool f64,
+                                  int cus)
 {
     constexpr int64_t kLds = 158 * 1024, kOneBlock = 96 * 1024, kCachedBytes = 64 * 1024;
     const int64_t entry = f64 ? 8 : 4, share = (f64 ? 48 : 16) * 1024, kb = m * n * entry;
@@ -54,7 +58,7 @@ inline ResidentPlan resident_plan(int model, int np, int nv, int64_t m, int64_t 
     int64_t P = kb <= kOneBlock && ne <= kResMaxElements
                     ? 1 : std::max<int64_t>(2, (kb + share - 1) / share);
     P = std::max<int64_t>(P, (ne + 55) / 56);
-    P = std::min<int64_t>(P, kResMaxBlocks);
+    P = std::min<int64_t>(P, std::max(1, std::min(cus, kResMaxBlocks)));
     // element boundaries at equal numbers of rows
     const bool ap = model == RES_MODEL_ANTIPLANE, ps = model == RES_MODEL_PLANESTRAIN;
     const int64_t rp = ps ? 2 : ap ? 1 : 3, rv = ps ? 3 : ap ? 2 : 6;

@@ -17,6 +17,7 @@ struct DevBuf {
 
 struct ucy_ctx {
     int device = 0;
+    int cus = 0;               // compute units of the device
     hipStream_t stream = nullptr;
     std::string err;
     // elastic moduli
