@@ -331,8 +331,9 @@ int ucy_rkqs(ucy_ctx *ctx, int n, double *t, double *y, double *dydt, const doub
 /* Main loop of ratestate.f90:307-328 run device-resident: many RK45 attempts
  * per launch of a resident kernel, or (K beyond 1 GB in binary64, 2 GB reduced,
  * or no room on the device for the resident blocks) one graph-captured attempt
- * per replay, with the same bits.  y is read at entry and written at exit.  Optional logs receive, per accepted step, the time reached, dt_done
- * and the vMax of the step-start odefun (ratestate.f90:530-532). */
+ * per replay, with the same bits.  y is read at entry and written at exit.
+ * Optional logs receive, per accepted step, the time reached, dt_done and the
+ * vMax of the step-start odefun (ratestate.f90:530-532). */
 typedef struct {
     double time;        /* simulated time reached */
     double dt_next;     /* next step size */
@@ -374,6 +375,21 @@ typedef struct {
 int ucy_integrate_ex(ucy_ctx *ctx, double *y, double t0, double interval, double dt0,
                      int64_t max_steps, double epsilon, double max_step,
                      const ucy_step_log *log, ucy_run_stats *stats);
+
+/* Limits of the resident kernel of ucy_integrate (no counterpart in the
+ * reference); results do not depend on them.  launches: launches of a call after
+ * which the captured attempt goes on; attempts: RK45 attempts per launch, at most
+ * those of some 30 ms (a launch holds the CUs' LDS meanwhile); wait_seconds: how
+ * long a block waits for other blocks' values before the call goes back to the
+ * launch's start and on with the captured attempt, at most the default's 2 s.
+ * Negative (attempts: or 0): the default, no limit of launches. */
+int ucy_set_resident_limits(ucy_ctx *ctx, int launches, int attempts, double wait_seconds);
+/* what the last ucy_integrate of the context did: launches of the resident kernel
+ * that counted, and why the captured attempt went on (0: it did not) */
+#define UCY_RESIDENT_NOT_PLANNED 1   /* the model's size, or displacement logging */
+#define UCY_RESIDENT_NO_ROOM 2       /* the blocks were not resident together in 2 ms */
+#define UCY_RESIDENT_WAIT 3          /* a wait for another block's values ran out */
+int ucy_resident_info(ucy_ctx *ctx, int *launches, int *left);
 
 /* Measurement hook (no counterpart in the reference): average duration in
  * seconds of the fused matvec + odefun post-pass kernel (the dominant kernel

@@ -15,7 +15,7 @@ run that ends in an error.
 import numpy as np
 import pytest
 
-from unicycle_amd import PREC_MIXED, PREC_SPLIT_BF16, UcyError, configs
+from unicycle_amd import PREC_F64, PREC_MIXED, PREC_SPLIT_BF16, UcyError, configs
 
 pytestmark = pytest.mark.gpu
 
@@ -204,4 +204,50 @@ def test_end_time_and_errors(engine_factory):
         eng.integrate(bad, HUGE, max_steps=5)
     again = eng.integrate(y, 5.0e5, max_step=1e5, log_cap=100)
     assert np.array_equal(again.y, r.y)
+    eng.close()
+
+
+# ---- the hand-over to the captured attempt ------------------------------------
+def _handed_over(eng, y, launches, attempts, wait, kw):
+    eng.set_resident_limits(launches, attempts, wait)
+    r = eng.integrate(y, HUGE, **kw)
+    info = eng.resident_info()
+    eng.set_resident_limits()
+    return r, info
+
+
+@pytest.mark.parametrize("precision", [PREC_F64, PREC_MIXED, PREC_SPLIT_BF16])
+@pytest.mark.parametrize("name", ["thrust-247", "volumes-39-200", "thrust-1081"])
+def test_a_wait_that_runs_out(engine_factory, name, precision):
+    """With no time to wait no block gets the others' first values: every block
+    leaves at the end of its first attempt, and the call goes back to where the
+    launch began."""
+    eng = MODELS[name](engine_factory)
+    eng.buildG(precision)
+    y = _start(eng)
+    kw = dict(max_steps=30, log_cap=30, history=True, observe=[0, y.size - 1], max_step=1e6)
+    want = eng.integrate(y, HUGE, **kw)
+    assert eng.resident_info()[0] >= 1 and eng.resident_info()[1] == 0
+    got, info = _handed_over(eng, y, -1, 0, 0.0, kw)
+    assert info == (0, 3)
+    _same(got, want)
+    _same(eng.integrate(y, HUGE, **kw), want)
+    eng.close()
+
+
+@pytest.mark.parametrize("precision", [PREC_F64, PREC_MIXED])
+@pytest.mark.parametrize("launches", [0, 1, 2, 3, 7])
+def test_no_room_after_some_launches(engine_factory, launches, precision):
+    """One attempt per launch: the captured attempt goes on after a step, and
+    after rejected attempts of a step."""
+    eng = MODELS["thrust-247"](engine_factory)
+    eng.buildG(precision)
+    y = _start(eng)
+    # the first step is rejected several times
+    kw = dict(dt0=1e8, epsilon=1e-9, max_steps=20, log_cap=20, history=True, observe=[0, 5])
+    want = eng.integrate(y, HUGE, **kw)
+    assert want.reject_log[0] >= 2 and eng.resident_info()[1] == 0
+    got, info = _handed_over(eng, y, launches, 1, -1.0, kw)
+    assert info == (launches, 2)
+    _same(got, want)
     eng.close()

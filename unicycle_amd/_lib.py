@@ -127,6 +127,8 @@ _SIGS = {
                            C.POINTER(RunStats)]),
     "ucy_integrate_ex": (_i, [_vp, _pd, _d, _d, _d, _i64, _d, _d, C.POINTER(StepLog),
                               C.POINTER(RunStats)]),
+    "ucy_set_resident_limits": (_i, [_vp, _i, _i, _d]),
+    "ucy_resident_info": (_i, [_vp, _pi, _pi]),
     "ucy_time_rhs_kernel": (_i, [_vp, _i, _pd]),
     "ucy_mlp_create": (_vp, [_vp, C.c_uint64]),
     "ucy_mlp_destroy": (None, [_vp]),

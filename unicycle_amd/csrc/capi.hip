@@ -237,8 +237,8 @@ extern "C" ucy_ctx *ucy_create(int device, int flags)
         delete c;
         return nullptr;
     }
-    if (hipHostMalloc((void **)&c->h_ctl, sizeof(Control), hipHostMallocDefault) != hipSuccess ||
-        hipMalloc((void **)&c->d_ctl, sizeof(Control)) != hipSuccess) {
+    if (hipHostMalloc((void **)&c->h_ctl, kControlBytes, hipHostMallocDefault) != hipSuccess ||
+        hipMalloc((void **)&c->d_ctl, kControlBytes) != hipSuccess) {
         delete c;
         return nullptr;
     }
@@ -1693,9 +1693,10 @@ static int plan_resident(ucy_ctx *c, const PlainDims &d, ResArgs &a, size_t &lds
     if (!plan.P) return 1;
     const int64_t P = plan.P;
     lds = plan.lds;
-    const size_t hb = 64, bb = 8 * (kResMaxBlocks / 2 + 1);
+    const size_t bb = (sizeof(int) * (kResMaxBlocks + 1) + 255) / 256 * 256;
     a.xbytes = 8 * 4 * (3 * (size_t)P + (size_t)d.n);
-    int rc = ensure_buf(c, c->res, hb + bb + a.xbytes);
+    const size_t sb = sizeof(double) * (3 * (size_t)d.dim + (size_t)d.n + (size_t)d.m);
+    int rc = ensure_buf(c, c->res, bb + a.xbytes + sb);
     if (rc) return rc;
     char *p = (char *)c->res.p;
     a.d = d;
@@ -1704,10 +1705,11 @@ static int plan_resident(ucy_ctx *c, const PlainDims &d, ResArgs &a, size_t &lds
     a.rh = c->d_rh;
     a.b = c->rb;
     a.ctl = c->d_ctl;
-    a.head = (ResHead *)p;
-    a.bounds = (const int *)(p + hb);
-    a.red = (unsigned long long *)(p + hb + bb);
+    a.head = resident_head(c->d_ctl);
+    a.bounds = (const int *)p;
+    a.red = (unsigned long long *)(p + bb);
     a.v = a.red + 4 * 3 * P;
+    a.saved = (double *)(p + bb + a.xbytes);
     a.P = plan.P;
     a.threads = P == 1 && d.m <= 8 ? 128 : kResThreads;
     a.el_max = plan.el_max;
@@ -1717,21 +1719,62 @@ static int plan_resident(ucy_ctx *c, const PlainDims &d, ResArgs &a, size_t &lds
     // launches of some 30 ms: 20 us and K's reading time per attempt
     const double us = 20.0 + (double)d.m * d.n * (f64 ? 8 : 4) / 1.0e6;
     a.max_attempts = (int)std::max(16.0, std::min(2000.0, 30000.0 / us));
+    if (c->res_limit_attempts > 0) a.max_attempts = std::min(a.max_attempts, c->res_limit_attempts);
+    a.form_ticks = 200000;     // 2 ms
+    a.wait_ticks = c->res_limit_wait < 0 ? 200000000ull    // 2 s
+                                         : (unsigned long long)(std::min(c->res_limit_wait, 2.0) * 1e8);
     HIPCHK(hipMemcpyAsync((void *)a.bounds, plan.bounds.data(), sizeof(int) * (P + 1),
                           hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));   // the plan is on this call's stack
     return 0;
 }
 
-// one launch of the resident integrator, the control block read back
-static int run_resident(ucy_ctx *c, const ResArgs &a, size_t lds)
+// one launch of the resident integrator, the control block and the head read back;
+// left: 0, or why the captured attempt has to go on from here (UCY_RESIDENT_*)
+static int run_resident(ucy_ctx *c, ResArgs &a, size_t lds, int &left)
 {
+    const Control before = *c->h_ctl;
+    if (c->res_limit_launches >= 0 && c->res_launches >= c->res_limit_launches)
+        a.form_ticks = 0;   // the blocks find no room
     HIPCHK(hipMemsetAsync(a.head, 0, sizeof(ResHead), c->stream));
     HIPCHK(hipMemsetAsync(a.red, 0xff, a.xbytes, c->stream));
     HIPCHK(launch_resident(c->stream, a, lds));
-    HIPCHK(hipMemcpyAsync(c->h_ctl, c->d_ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(c->h_ctl, c->d_ctl, kControlBytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    const ResHead &head = *resident_head(c->h_ctl);
+    left = head.failed ? UCY_RESIDENT_WAIT : head.state != 1 ? UCY_RESIDENT_NO_ROOM : 0;
+    if (!head.failed) {
+        c->res_launches += left == 0;
+        return 0;
+    }
+    // a wait ran out: back to what the launch found (neighbours in the work buffers)
+    const RkBuffers &b = c->rb;
+    *c->h_ctl = before;
+    HIPCHK(hipMemcpyAsync(c->d_ctl, c->h_ctl, sizeof(Control), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(b.y, a.saved, sizeof(double) * 3 * a.d.dim, hipMemcpyDeviceToDevice,
+                          c->stream));
+    if (b.v0)
+        HIPCHK(hipMemcpyAsync(b.v0, a.saved + 3 * (size_t)a.d.dim,
+                              sizeof(double) * ((size_t)a.d.n + a.d.m), hipMemcpyDeviceToDevice,
+                              c->stream));
     return 0;
+}
+
+extern "C" int ucy_set_resident_limits(ucy_ctx *c, int launches, int attempts, double wait_seconds)
+{
+    if (!c || !(wait_seconds == wait_seconds)) return UCY_ERR_ARG;
+    c->res_limit_launches = launches;
+    c->res_limit_attempts = attempts;
+    c->res_limit_wait = wait_seconds;
+    return UCY_OK;
+}
+
+extern "C" int ucy_resident_info(ucy_ctx *c, int *launches, int *left)
+{
+    if (!c) return UCY_ERR_ARG;
+    if (launches) *launches = c->res_launches;
+    if (left) *left = c->res_left;
+    return UCY_OK;
 }
 
 extern "C" int ucy_integrate(ucy_ctx *c, double *y, double interval, double dt0,
@@ -1850,21 +1893,17 @@ extern "C" int ucy_integrate_ex(ucy_ctx *c, double *y, double t0, double interva
     HIPCHK(hipMemcpyAsync(b.y, y, sizeof(double) * d.dim, hipMemcpyHostToDevice, c->stream));
     ResArgs ra{};
     size_t res_lds = 0;
+    c->res_launches = 0;
     rc = want_disp ? 1 : plan_resident(c, d, ra, res_lds);
-    bool resident = rc == 0;
+    c->res_left = rc ? UCY_RESIDENT_NOT_PLANNED : 0;
     if (rc > 0) rc = capture_attempt(c);
     auto w0 = std::chrono::steady_clock::now();
     int batch = 16;
     while (rc == 0) {
-        if (resident) {
-            const long long before = h.attempts;
-            rc = run_resident(c, ra, res_lds);
-            if (rc || h.done) break;
-            // the blocks found no room together: the captured attempt goes on
-            if (h.attempts == before) {
-                resident = false;
-                rc = capture_attempt(c);
-            }
+        if (!c->res_left) {
+            rc = run_resident(c, ra, res_lds, c->res_left);
+            if (rc || (!c->res_left && h.done)) break;
+            if (c->res_left) rc = capture_attempt(c);
             continue;
         }
         for (int i = 0; i < batch; i++) HIPCHK(hipGraphLaunch(c->graph, c->stream));
@@ -1955,7 +1994,6 @@ extern "C" int ucy_integrate_ex(ucy_ctx *c, double *y, double t0, double interva
     }
     if (h.error == 1) return fail(c, UCY_ERR_UNDERFLOW, "stepsize underflow in RKQS");
     if (h.error == 2) return fail(c, UCY_ERR_NONFINITE, "non-finite error norm");
-    if (h.error == 3) return fail(c, UCY_ERR_HIP, "resident integrator: a block did not answer");
     return UCY_OK;
 }
 

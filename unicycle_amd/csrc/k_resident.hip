@@ -44,7 +44,11 @@
 // All blocks have to be resident before the first exchange.  They count
 // themselves in; if they are not complete within 2 ms (another kernel holds
 // the CUs), all of them leave before anything has changed, and the caller
-// falls back on the captured attempt.  The later waits are bounded too.
+// falls back on the captured attempt.  The later waits are bounded too, by 2 s: a
+// block whose wait runs out raises a flag for the host and for the others' waits,
+// and takes part until the attempt's end, where it leaves.  The launch's results
+// are then void: the host puts back the state that the launch found, which every
+// block has kept a copy of, and goes on with the captured attempt.
 //
 // The row sums keep wave_rows_dot's order and the element arithmetic is the
 // captured attempt's (ode_dev.h): a run gives the same bits on either.
@@ -67,8 +71,6 @@ __device__ __forceinline__ void agent_store(T *p, T v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-constexpr unsigned long long kFormTicks = 200000;     // 2 ms of the 100 MHz clock
-constexpr unsigned long long kWaitTicks = 200000000;  // 2 s
 constexpr unsigned long long kEmpty = ~0ull;
 
 // the bits of a value that is to be exchanged: never kEmpty
@@ -224,7 +226,7 @@ resident_kernel(ResArgs a)
     constexpr int NSM = ResModel<M>::ns, NVM = ResModel<M>::nv, NTM = ResModel<M>::nt;
     extern __shared__ __attribute__((aligned(16))) double lds[];
     __shared__ Control ctl;
-    __shared__ int formed, stop, go;
+    __shared__ int formed, stop, go, leave;
     const PlainDims &d = a.d;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, T = blockDim.x, nw = T >> 6;
     const int P = a.P, blk = blockIdx.x;
@@ -233,12 +235,12 @@ resident_kernel(ResArgs a)
     if (t == 0) {
         formed = 1;
         if (P > 1) {
-            if (atomicAdd(&a.head->arrived, 1u) == (unsigned)P - 1)
+            if (atomicAdd(&a.head->arrived, 1u) == (unsigned)P - 1 && a.form_ticks)
                 atomicCAS(&a.head->state, 0u, 1u);
             const unsigned long long t0 = wall_clock64();
             unsigned s;
             while ((s = agent_load(&a.head->state)) == 0) {
-                if (wall_clock64() - t0 > kFormTicks) atomicCAS(&a.head->state, 0u, 2u);
+                if (wall_clock64() - t0 >= a.form_ticks) atomicCAS(&a.head->state, 0u, 2u);
                 __builtin_amdgcn_s_sleep(1);
             }
             formed = s == 1;
@@ -246,7 +248,7 @@ resident_kernel(ResArgs a)
             a.head->state = 1;
         }
         ctl = *a.ctl;
-        stop = 0;
+        stop = leave = 0;
     }
     __syncthreads();
     if (!formed) return;
@@ -295,19 +297,21 @@ resident_kernel(ResArgs a)
 #pragma unroll
     for (int k = 0; k < NVM; k++) v0[k] = vp[k] = 0.0;
     if (mine) {
+        double *const sy = a.saved, *const sd = sy + d.dim, *const ss = sd + d.dim;
         if (!vol) f = a.fr[e];
 #pragma unroll
         for (int k = 0; k < NSM; k++)
             if (k < ns) {
-                y[k] = p[k] = a.b.y[so + k];
-                scale(k) = a.b.yscal[so + k];
-                dydt(k) = a.b.dydt[so + k];
+                sy[so + k] = y[k] = p[k] = a.b.y[so + k];
+                ss[so + k] = scale(k) = a.b.yscal[so + k];
+                sd[so + k] = dydt(k) = a.b.dydt[so + k];
             }
         if (red_prec && !ctl.need_rhs) {
+            double *const sv = ss + d.dim, *const st0 = sv + n;
 #pragma unroll
             for (int k = 0; k < NVM; k++)
-                if (k < nv) v0[k] = a.b.v0[vo + k];
-            for (int k = 0; k < nt; k++) t0L[ro + k] = a.b.t0[r0 + ro + k];
+                if (k < nv) sv[vo + k] = v0[k] = a.b.v0[vo + k];
+            for (int k = 0; k < nt; k++) st0[r0 + ro + k] = t0L[ro + k] = a.b.t0[r0 + ro + k];
         }
     }
     __syncthreads();
@@ -355,15 +359,18 @@ resident_kernel(ResArgs a)
         }
         if (mine) elem_early<M>(vol, p, f, q);
     };
-    // polls one entry; a wait that runs into its limit ends the run
+    // polls one entry; a wait that runs into its limit, or is behind one that has,
+    // ends the block's part in the run
     auto poll = [&](const unsigned long long *x) {
         unsigned long long b, t0 = 0;
         for (int spin = 1; (b = agent_load(x)) == kEmpty; spin++)
-            if ((spin & 1023) == 0) {
+            if ((spin & 1023) == 0 || a.wait_ticks == 0) {
                 const unsigned long long now = wall_clock64();
                 if (!t0) t0 = now;
-                if (now - t0 > kWaitTicks || *(volatile int *)&stop) {
+                if (now - t0 >= a.wait_ticks || *(volatile int *)&stop ||
+                    agent_load(&a.head->failed)) {
                     stop = 1;
+                    agent_store(&a.head->failed, 1u);
                     return 0ull;
                 }
             }
@@ -467,13 +474,14 @@ resident_kernel(ResArgs a)
 
     // ---- the workers --------------------------------------------------------
     // They and wave 0 go through the same barriers: per exchange one when the
-    // slip rates are in LDS, one when K v is.
+    // slip rates are in LDS, one when K v is.  Nobody polls between the two of a
+    // step start, where wave 0 reads `stop` into `leave`: all waves leave alike.
     if (w != 0) {
         // 1: the call's first step start; 2..6: a stage; 7: an attempt's end,
         // with the next step's start if the step is accepted
         int phase = ctl.need_rhs && !ctl.done ? 1 : 2;
         for (int att = 0;;) {
-            if (phase == 2 && !(att < a.max_attempts && !ctl.done && !stop)) break;
+            if (phase == 2 && !(att < a.max_attempts && !ctl.done && !leave)) break;
             collect();
             __syncthreads();
             const bool start = phase == 1 || phase == 7;
@@ -498,12 +506,13 @@ resident_kernel(ResArgs a)
         if (lane == 0) {
             ctl.vmax = __longlong_as_double((long long)bv);
             ctl.emax = __longlong_as_double((long long)bn);
+            leave = stop;
         }
         __syncthreads();
         fresh = true;
     }
 
-    for (int att = 0; att < a.max_attempts && !ctl.done && !stop; att++) {
+    for (int att = 0; att < a.max_attempts && !ctl.done && !leave; att++) {
         const double h = ctl.h;
         if (mine) {
             if (fresh) {   // a new step: dydt and yscal (ratestate.f90:309-315)
@@ -585,6 +594,7 @@ resident_kernel(ResArgs a)
         if (lane == 0) {
             ctl.errmax_bits = be;
             controller_step(a.b, &ctl, blk == 0);
+            leave = stop;
             if (ctl.accepted) {
                 ctl.vmax = __longlong_as_double((long long)bv);
                 ctl.emax = __longlong_as_double((long long)bn);
@@ -631,10 +641,6 @@ resident_kernel(ResArgs a)
         if (ctl.need_rhs) {    // formed again by the next step start
             ctl.vmax = 0.0;
             ctl.emax = 0.0;
-        }
-        if (stop) {
-            ctl.error = 3;
-            ctl.done = 1;
         }
         *a.ctl = ctl;
     }

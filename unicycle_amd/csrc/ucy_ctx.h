@@ -82,8 +82,13 @@ struct ucy_ctx {
     hipGraphExec_t graph = nullptr;
     // scratch for the per-kernel hooks
     DevBuf hook;
-    // the resident integrator's exchange buffers
+    // the resident integrator's exchange buffers and its copy of the state
     DevBuf res;
+    // its limits (ucy_set_resident_limits; < 0: the default) and what the last
+    // ucy_integrate did (ucy_resident_info)
+    int res_limit_launches = -1, res_limit_attempts = -1;
+    double res_limit_wait = -1.0;
+    int res_launches = 0, res_left = 0;
     // ensembles created on this context (destroyed with it)
     std::vector<struct ucy_ensemble *> ensembles;
 };

@@ -402,6 +402,22 @@ class Engine:
         res.emax_log = cut(logs[5])
         return res
 
+    def set_resident_limits(self, launches: int = -1, attempts: int = -1,
+                            wait_seconds: float = -1.0):
+        """Limits of integrate's resident kernel (negative: the default): launches
+        of a call, attempts per launch, seconds that a block waits for another's
+        values.  The captured attempt goes on beyond them, with the same bits."""
+        self._chk(self._L.ucy_set_resident_limits(self._h, int(launches), int(attempts),
+                                                  float(wait_seconds)))
+
+    def resident_info(self):
+        """(launches, left) of the last integrate: launches of the resident kernel,
+        and why the captured attempt went on: 0 it did not, 1 the model's size or
+        displacement logging, 2 no room on the device, 3 a wait ran out."""
+        n, left = C.c_int(), C.c_int()
+        self._chk(self._L.ucy_resident_info(self._h, C.byref(n), C.byref(left)))
+        return n.value, left.value
+
     def time_rhs_kernel(self, iters: int = 50) -> float:
         """Average seconds of the fused matvec + post-pass kernel (HIP events)."""
         out = C.c_double()
