@@ -207,6 +207,28 @@ def test_end_time_and_errors(engine_factory):
     eng.close()
 
 
+@pytest.mark.parametrize("name", ["antiplane-1", "thrust-247", "volumes-large",
+                                  "planestrain-volumes", "thrust-1081"])
+def test_every_entry_observed(engine_factory, name):
+    """All entries in a shuffled order, some of them three times, and at next to no
+    cost: the time per attempt without observed entries, and half as much for the
+    stores (measured: 6 % at most; 11 to 30 times when every lane looked through
+    the whole list)."""
+    eng = MODELS[name](engine_factory)
+    eng.buildG()
+    y = _start(eng)
+    eng.buildO(np.array([[1e3, 2e3, 0.0]]))
+    rng = np.random.default_rng(5)
+    obs = rng.permutation(np.concatenate([np.arange(y.size), [0, 0, y.size - 1, y.size // 2]]))
+    kw = dict(max_steps=60, log_cap=60, history=True)
+    _same(eng.integrate(y, HUGE, observe=obs, **kw),
+          eng.integrate(y, HUGE, observe=obs, displacement=True, **kw))
+    few, many = (min(eng.integrate(y, HUGE, observe=o, **kw).wall_seconds for _ in range(5))
+                 for o in ([0], obs))
+    assert many < 1.5 * few + 1e-3
+    eng.close()
+
+
 # ---- the hand-over to the captured attempt ------------------------------------
 def _handed_over(eng, y, launches, attempts, wait, kw):
     eng.set_resident_limits(launches, attempts, wait)

@@ -1686,17 +1686,19 @@ static int capture_attempt(ucy_ctx *c)
 
 // The resident integrator's plan (resident_plan.h) with its buffers in place.
 // 0: planned; 1: the model takes the captured attempt; < 0: an error.
-static int plan_resident(ucy_ctx *c, const PlainDims &d, ResArgs &a, size_t &lds)
+static int plan_resident(ucy_ctx *c, const PlainDims &d, int64_t n_obs, const int64_t *obs,
+                         ResArgs &a, size_t &lds)
 {
     const bool f64 = c->kprec == UCY_PREC_F64;
     const ResidentPlan plan = resident_plan(c->model, d.np, d.nv, d.m, d.n, f64, c->cus);
-    if (!plan.P) return 1;
+    if (!plan.P || n_obs >= kResMore) return 1;
     const int64_t P = plan.P;
     lds = plan.lds;
     const size_t bb = (sizeof(int) * (kResMaxBlocks + 1) + 255) / 256 * 256;
     a.xbytes = 8 * 4 * (3 * (size_t)P + (size_t)d.n);
     const size_t sb = sizeof(double) * (3 * (size_t)d.dim + (size_t)d.n + (size_t)d.m);
-    int rc = ensure_buf(c, c->res, bb + a.xbytes + sb);
+    const size_t ob = sizeof(int) * (n_obs > 0 ? (size_t)d.dim + (size_t)n_obs : 0);
+    int rc = ensure_buf(c, c->res, bb + a.xbytes + sb + ob);
     if (rc) return rc;
     char *p = (char *)c->res.p;
     a.d = d;
@@ -1725,7 +1727,15 @@ static int plan_resident(ucy_ctx *c, const PlainDims &d, ResArgs &a, size_t &lds
                                          : (unsigned long long)(std::min(c->res_limit_wait, 2.0) * 1e8);
     HIPCHK(hipMemcpyAsync((void *)a.bounds, plan.bounds.data(), sizeof(int) * (P + 1),
                           hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));   // the plan is on this call's stack
+    std::vector<int> columns(ob / sizeof(int));
+    if (n_obs > 0) {
+        int *dev = (int *)(p + bb + a.xbytes + sb);
+        resident_observed(d.dim, n_obs, obs, columns.data(), columns.data() + d.dim);
+        a.obs_col = dev;
+        a.obs_next = dev + d.dim;
+        HIPCHK(hipMemcpyAsync(dev, columns.data(), ob, hipMemcpyHostToDevice, c->stream));
+    }
+    HIPCHK(hipStreamSynchronize(c->stream));   // plan and columns are on this call's stack
     return 0;
 }
 
@@ -1894,7 +1904,7 @@ extern "C" int ucy_integrate_ex(ucy_ctx *c, double *y, double t0, double interva
     ResArgs ra{};
     size_t res_lds = 0;
     c->res_launches = 0;
-    rc = want_disp ? 1 : plan_resident(c, d, ra, res_lds);
+    rc = want_disp ? 1 : plan_resident(c, d, n_obs, log ? log->obs_index : nullptr, ra, res_lds);
     c->res_left = rc ? UCY_RESIDENT_NOT_PLANNED : 0;
     if (rc > 0) rc = capture_attempt(c);
     auto w0 = std::chrono::steady_clock::now();

@@ -604,16 +604,20 @@ resident_kernel(ResArgs a)
         if (fresh && mine) {
             // the export of the step-start entries (ratestate.f90:488-536)
             const int64_t row = ctl.log_count - 1;
-            if (row >= 0 && row < ctl.log_cap)
-                for (int64_t j = 0; j < a.b.n_obs; j++) {
-                    const int64_t i = a.b.obs_idx[j] - so;
+            if (a.b.n_obs > 0 && row >= 0 && row < ctl.log_cap) {
+                double *oy = a.b.obs_y + row * a.b.n_obs, *od = a.b.obs_dydt + row * a.b.n_obs;
+                int col[NSM];
 #pragma unroll
-                    for (int k = 0; k < NSM; k++)
-                        if (k < ns && i == k) {
-                            a.b.obs_y[row * a.b.n_obs + j] = y[k];
-                            a.b.obs_dydt[row * a.b.n_obs + j] = dydt(k);
-                        }
-                }
+                for (int k = 0; k < NSM; k++) col[k] = k < ns ? a.obs_col[so + k] : -1;
+#pragma unroll
+                for (int k = 0; k < NSM; k++)
+                    for (int v = col[k]; v >= 0;) {
+                        const int j = v & ~kResMore;
+                        oy[j] = y[k];
+                        od[j] = dydt(k);
+                        v = v & kResMore ? a.obs_next[j] : -1;
+                    }
+            }
 #pragma unroll
             for (int k = 0; k < NSM; k++) y[k] = p[k];
         }

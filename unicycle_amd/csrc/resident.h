@@ -39,6 +39,9 @@ struct ResArgs {
     unsigned long long *v;            // [4][n] slip rates
     size_t xbytes;                    // of red and v together
     const int *bounds;                // [P + 1] first element of each block
+    // columns of the log of observed entries (b.n_obs > 0): per state entry one, or
+    // -1; with kResMore set another follows, in obs_next at the column
+    const int *obs_col, *obs_next;
     int P, threads;
     int el_max, rows_max;             // largest share of a block, both even
     int rows_lds;                     // rows of a block kept in LDS
