@@ -85,3 +85,21 @@ def test_shallow_splits(engine_factory, nx, nz, precision, bound):
         assert np.all(np.abs(ens.matvec(0, V) - want) <= bound * scale), kb
     ens.close()
     eng.close()
+
+
+@pytest.mark.parametrize("precision", [PREC_F64, PREC_BF16_I8])
+def test_equal_splits_are_timed_once(engine_factory, precision):
+    """Depths that split K alike are one launch and share one timing: a build times
+    each launch once, whatever the number of depths."""
+    eng = engine_factory()
+    for nx, nz in ((8, 4), (24, 12)):
+        ens, y0s = _ensemble(eng, precision, [(nx, nz)], 8)
+        nkb = -(-2 * y0s[0][0].n // 16)
+        table = ens.tuning()[2].reshape(-1, 11)
+        splits = [-(-nkb // kb) for kb in (32, 48, 64, 80, 96, 104, 128, 160, 192, 256, 512)]
+        assert np.any(table > 0)
+        for row in table:
+            for s in set(splits):
+                assert len({t for t, k in zip(row, splits) if k == s}) == 1
+        ens.close()
+    eng.close()
