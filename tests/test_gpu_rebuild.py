@@ -1,5 +1,5 @@
-"""Assemblies into a kernel that the context holds already: same shape, another
-shape of the same size, another precision; bit-identical to a fresh context's."""
+"""Assemblies into a kernel that the context holds already: another geometry of the
+same shape, other shapes, another precision; bit-identical to a fresh context's."""
 import numpy as np
 import pytest
 

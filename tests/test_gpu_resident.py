@@ -7,11 +7,15 @@ error ratios, rejections and observed entries.  A run that also logs an
 observation point's displacement takes the captured attempt; without it, a
 kernel of this size takes the resident one.
 
-Sizes: one element; one block and the first two-block size; blocks' shares that
+Sizes: one element; the largest models of one block (56 segments, 45 patches) and
+the next ones, of two and three; blocks' shares that
 do not divide; rows that do not fit the blocks' LDS; every model, with volumes;
 the reduced forms of K; a run split into calls; an end time, a step limit and a
-run that ends in an error.
+run that ends in an error; observed entries; two runs at once; the hand-over to the
+captured attempt at the start, between launches and after a wait that ran out.
 """
+import threading
+
 import numpy as np
 import pytest
 
@@ -80,6 +84,8 @@ def _planestrain(make, n, n2=0, n3=0):
 MODELS = {
     "antiplane-1": lambda mk: _segments(mk, 1),
     "antiplane-2": lambda mk: _segments(mk, 2),
+    "antiplane-56": lambda mk: _segments(mk, 56),
+    "antiplane-57": lambda mk: _segments(mk, 57),
     "antiplane-64": lambda mk: _segments(mk, 64),
     "antiplane-65": lambda mk: _segments(mk, 65),
     "antiplane-111": lambda mk: _segments(mk, 111),
@@ -87,6 +93,7 @@ MODELS = {
     "thrust-1": lambda mk: _thrust(mk, 1, 1),
     "thrust-44": lambda mk: _thrust(mk, 11, 4),
     "thrust-45": lambda mk: _thrust(mk, 9, 5),
+    "thrust-46": lambda mk: _thrust(mk, 23, 2),
     "thrust-247": lambda mk: _thrust(mk, 19, 13),
     "thrust-1081": lambda mk: _thrust(mk, 47, 23),
     "thrust-2816": lambda mk: _thrust(mk, 64, 44),
@@ -273,3 +280,30 @@ def test_no_room_after_some_launches(engine_factory, launches, precision):
     assert info == (launches, 2)
     _same(got, want)
     eng.close()
+
+
+@pytest.mark.parametrize("name", ["thrust-247", "thrust-1081", "volumes-39-200"])
+def test_two_contexts_at_once(engine_factory, name):
+    """Two runs share the device's CUs, or take turns at them (256 blocks of nearly
+    all LDS, several launches each), or leave them for the captured attempt."""
+    engs = [MODELS[name](engine_factory) for _ in range(2)]
+    for e in engs:
+        e.buildG()
+    y = _start(engs[0])
+    kw = dict(max_steps=300, log_cap=300, history=True, observe=[0, 3])
+    for e in engs:
+        e.set_resident_limits(attempts=40)
+    want = engs[0].integrate(y, HUGE, **kw)
+    got = [None, None]
+
+    def run(i):
+        got[i] = engs[i].integrate(y, HUGE, **kw)
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g in got:
+        _same(g, want)
+    for e in engs:
+        e.close()

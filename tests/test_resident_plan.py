@@ -104,3 +104,4 @@ def test_limits(plan):
     assert plan(0, 4096, 0, True)[2] == 256 and plan(0, 4800, 0, True)[2] == 0
     assert plan(0, 8192, 0, False)[2] == 256 and plan(0, 10000, 0, False)[2] == 0
     assert plan(1, 56, 0, True)[2] == 1 and plan(1, 57, 0, True)[2] == 2
+    assert plan(0, 45, 0, True)[2] == 1 and plan(0, 46, 0, True)[2] == 3
