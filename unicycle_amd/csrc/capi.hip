@@ -678,8 +678,9 @@ extern "C" int ucy_build_kernel(ucy_ctx *c, int precision)
     }
     free_work(c);
     // A kernel of the same shape is written over: mapping and unmapping 137 MB
-    // took 0.2 ms of an assembly of 0.57 ms, at times 3 ms.  What else reads it,
-    // on any stream, has ended then, as it had when hipFree returned.
+    // took 0.2 ms of an assembly of 0.57 ms, at times 3 ms.  (A context's first
+    // assembly maps it, 0.1 ms.)  What else reads it, on any stream, has ended then,
+    // as it had when hipFree returned.
     if (c->K && (c->m != m || c->n != n)) {
         HIPCHK(hipFree(c->K));
         c->K = nullptr;

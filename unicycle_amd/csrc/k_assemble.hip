@@ -45,10 +45,10 @@ __device__ __forceinline__ void proj_volume(const Receiver &R, const double S[6]
 }
 
 // Bound by binary64 arithmetic and its latencies: 5.0 thousand instructions per
-// wave of pairs, 71 % of the issue slots.  Two waves per SIMD (28 registers to scratch) hide more than
-// they cost: 2048 sources on themselves take 0.85 ms, at one wave (276 registers)
-// 0.94, and with divisions in place of the corrected reciprocals of okada_dev.h
-// 1.09 and 1.30.
+// wave of pairs, 71 % of the issue slots.  Two waves per SIMD (28 registers to
+// scratch) hide more than they cost: 2048 sources on themselves take 0.74 ms, at one
+// wave (276 registers) 0.94, and with divisions in place of the corrected
+// reciprocals of okada_dev.h 1.09 and 1.30.
 template <int KIND>
 __global__ void __launch_bounds__(256, 2)
 okada_rows_kernel(OkadaMedium M, const OkadaSource *__restrict__ src, int ns,

@@ -232,8 +232,9 @@ tri_hook_kernel(TriMedium M, const TriSource *__restrict__ src, int ns,
 // the scalar unit and leave the vector registers to the derivatives (368, one
 // wave per SIMD).  2952 triangles, with the preparation of the sources on the host
 // (1.4 of it): 5.1 ms; with a source per lane 6.3 ms; with full gradients in the
-// source's frame, 512 registers and 1.2 KB of spills per lane 15.5 ms.  Forming the harmonic terms once per column fits two waves per
-// SIMD with 57 registers spilled and takes 5.9 ms.  The block's tile goes
+// source's frame, 512 registers and 1.2 KB of spills per lane 15.5 ms.  Forming the
+// harmonic terms once per column fits two waves per SIMD with 57 registers spilled
+// and takes 5.9 ms.  The block's tile goes
 // through LDS, so that a row is written in runs of 64 spw bytes.
 template <int KIND>
 __global__ void __launch_bounds__(256)

@@ -28,7 +28,7 @@ struct Rheology {
     double Gm, arr;
 };
 
-// Device-side control block of the graph-captured integrator.
+// Device-side control block of the captured and the resident integrator.
 struct Control {
     double time;        // simulated time (ratestate.f90:176,321)
     double h;           // step size of the next attempt (dt_try, or shrunk h)
@@ -178,7 +178,8 @@ void launch_obs_log(hipStream_t st, const RkBuffers &b, Control *ctl);
 // the attempt that accepted a step.
 void launch_disp_gemv(hipStream_t st, const double *O, int64_t rows, int64_t n, int np, int model,
                       const double *y, double *d, double *df, double *dl, const Control *ctl);
-// standalone Cash-Karp combination kernels for the ucy_rkck entry point
+// a whole Cash-Karp evaluation (ode45.f90:116-202) from b.y and b.dydt to b.ycand and
+// b.yerr, for ucy_rkck and ucy_rkqs
 void launch_rkck(hipStream_t st, const PlainDims &d, const double *K, const Friction *fr,
                  const Rheology *rh, RkBuffers b, double h);
 
