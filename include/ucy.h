@@ -394,8 +394,8 @@ int ucy_resident_info(ucy_ctx *ctx, int *launches, int *left);
 /* Measurement hook (no counterpart in the reference): average duration in
  * seconds of the fused matvec + odefun post-pass kernel (the dominant kernel
  * of every RHS), timed with HIP events on the context stream over iters
- * launches at the state of the last ucy_odefun call (or the last stage of
- * ucy_integrate). */
+ * launches on the work buffers as they are: the state of the last ucy_odefun,
+ * ucy_rkck or captured attempt (the resident kernel leaves them alone). */
 int ucy_time_rhs_kernel(ucy_ctx *ctx, int iters, double *avg_seconds);
 
 /* ---- batched ensembles (no counterpart in the reference) --------------- */
